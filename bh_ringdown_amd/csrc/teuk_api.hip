@@ -21,11 +21,21 @@ using namespace teuk;
 
 struct teuk_batch;
 
+// Longest a resident launch waits for all of its blocks to be on the GPU (s).
+constexpr double kResidentWait = 0.25;
+
 struct teuk_solver {
   teuk_params P;
   Grid g;
   DevState d;
   Tiling tiling;
+  // Resident stepping (teuk_resident.inc), unless the grid does not fit on
+  // the chip, a launch shape was set for the stage kernels, or a launch gave up.
+  bool resident = false;
+  ResShape res_shape{0, 0, 0};
+  double res_wait = kResidentWait;
+  int gate = 0;                  // which of the control block's two gates is next
+  bool res_pending = false;      // resident launches since the control block was last read
   teuk_batch *batch = nullptr;   // set while a batch drives this solver
   hipStream_t stream = nullptr;
   int nt = 0;              // scheduled steps: (int)(T/dt), body.cu:59
@@ -37,6 +47,7 @@ struct teuk_solver {
   // Kernel timing.
   bool timing = false;
   std::vector<hipEvent_t> ev;   // pairs
+  std::vector<int> ev_stages;   // stages between each pair
   size_t ev_used = 0;
   long long timed_launches = 0;
   double timed_ms = 0.0;
@@ -117,6 +128,59 @@ int validate(const teuk_params *p) {
 
 int scheduled_steps(const teuk_params *p) { return (int)(p->T / p->dt); }
 
+// Resident launches need all their blocks on the GPU at once, so within a
+// process each follows the one before it, whatever streams they are on: a
+// launch on another stream than the last one's first waits for the event
+// recorded behind that.  One chain per device.  (Other processes' launches
+// can still hold CUs; the launch's own gate bounds that wait.)
+struct ResidentChain {
+  std::mutex lock;
+  hipEvent_t done = nullptr;
+  hipStream_t last = nullptr;
+};
+constexpr int kMaxDevices = 64;
+ResidentChain g_chain[kMaxDevices];
+
+template <class Launch>
+int resident_launch(hipStream_t stream, Launch launch) {
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return TEUK_EHIP;
+  ResidentChain &c = g_chain[dev];
+  std::lock_guard<std::mutex> hold(c.lock);
+  if (!c.done) HIPCHK(hipEventCreateWithFlags(&c.done, hipEventDisableTiming));
+  if (c.last && c.last != stream) HIPCHK(hipStreamWaitEvent(stream, c.done, 0));
+  HIPCHK(launch());
+  HIPCHK(hipEventRecord(c.done, stream));
+  c.last = stream;
+  return TEUK_OK;
+}
+
+// A stream about to be destroyed (idle): the chain's event has completed, and
+// a new stream may get its handle.
+void chain_forget(hipStream_t stream) {
+  for (ResidentChain &c : g_chain) {
+    std::lock_guard<std::mutex> hold(c.lock);
+    if (c.last == stream) c.last = nullptr;
+  }
+}
+
+long long wait_ticks(double seconds) { return seconds > 0.0 ? (long long)(seconds * 1e8) + 1 : 0; }
+
+// CUs of the current device (asked of the runtime once per device).
+int device_cus() {
+  static std::mutex lock;
+  static int cus[kMaxDevices];
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  std::lock_guard<std::mutex> hold(lock);
+  if (!cus[dev]) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    cus[dev] = n;
+  }
+  return cus[dev];
+}
+
 // Kernel launches per step that the timing events cover as "stages": the
 // RK stages, or the staggered scheme's half and full step.
 int stages_per_step(int integrator) { return integrator == 0 ? 3 : (integrator == 1 ? 4 : 2); }
@@ -132,10 +196,34 @@ void flush_timing(teuk_solver *s) {
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, s->ev[i], s->ev[i + 1]) == hipSuccess) {
       s->timed_ms += ms;
-      s->timed_launches += stages_per_step(s->P.integrator);
+      s->timed_launches += s->ev_stages[i / 2];
     }
   }
   s->ev_used = 0;
+}
+
+// An event pair around back-to-back launches of `stages` stages (an event
+// between two launches would add its own gap to both).
+hipError_t timing_begin(teuk_solver *s, int stages) {
+  if (s->ev_used + 2 > s->ev.size()) {
+    if (s->ev.size() < 4096) {
+      for (int i = 0; i < 64; i++) {
+        hipEvent_t e;
+        const hipError_t err = hipEventCreate(&e);
+        if (err != hipSuccess) return err;
+        s->ev.push_back(e);
+      }
+      s->ev_stages.resize(s->ev.size() / 2);
+    } else {
+      flush_timing(s);
+    }
+  }
+  s->ev_stages[s->ev_used / 2] = stages;
+  return hipEventRecord(s->ev[s->ev_used], s->stream);
+}
+hipError_t timing_end(teuk_solver *s) {
+  s->ev_used += 2;
+  return hipEventRecord(s->ev[s->ev_used - 1], s->stream);
 }
 
 // One time step whose index is (device step counter + k_rel): source patches
@@ -147,34 +235,82 @@ int enqueue_step(teuk_solver *s, int k_rel) {
   // from one launch at the first step of each group of kRing steps (kRing
   // half steps for the staggered scheme)
   const int group = s->g.stag ? kRing / 2 : kRing;
-  if (s->has_src && k_rel % group == 0) HIPCHK(launch_source(s->g, s->d, k_rel, kRing, s->stream));
-  // Timing: one event pair around the step's back-to-back stage launches
-  // (an event between two launches would add its own gap to both).
-  if (s->timing) {
-    if (s->ev_used + 2 > s->ev.size()) {
-      if (s->ev.size() < 4096) {
-        for (int i = 0; i < 64; i++) {
-          hipEvent_t e;
-          HIPCHK(hipEventCreate(&e));
-          s->ev.push_back(e);
-        }
-      } else {
-        flush_timing(s);
-      }
-    }
-    HIPCHK(hipEventRecord(s->ev[s->ev_used], s->stream));
-  }
+  if (s->has_src && k_rel % group == 0) HIPCHK(launch_source(s->g, s->d, k_rel, kRing, false, run_stream(s)));
+  if (s->timing) HIPCHK(timing_begin(s, nstage));
   if (s->g.stag) {
-    HIPCHK(launch_so2_step(s->g, s->d, s->has_src, k_rel, s->stream));
+    HIPCHK(launch_so2_step(s->g, s->d, s->has_src, k_rel, run_stream(s)));
   } else {
     for (int st = 1; st <= nstage; st++)
-      HIPCHK(launch_stage(s->g, s->d, s->P.integrator, st, s->has_src, k_rel, s->tiling, s->stream));
+      HIPCHK(launch_stage(s->g, s->d, s->P.integrator, st, s->has_src, k_rel, s->tiling, run_stream(s)));
   }
-  if (s->timing) {
-    HIPCHK(hipEventRecord(s->ev[s->ev_used + 1], s->stream));
-    s->ev_used += 2;
+  if (s->timing) HIPCHK(timing_end(s));
+  return TEUK_OK;
+}
+
+// n steps by the per-stage launches, closed by the sentinel and the records.
+int stage_steps(teuk_solver *s, int n) {
+  if (n <= 0) return TEUK_OK;
+  for (int i = 0; i < n; i++) {
+    const int rc = enqueue_step(s, i);
+    if (rc) return rc;
+  }
+  HIPCHK(launch_sentinel(s->g, s->d, run_stream(s)));
+  HIPCHK(launch_finalize(s->g, s->d, n, nullptr, nullptr, run_stream(s)));
+  return TEUK_OK;
+}
+
+// n steps by resident launches of up to kRing steps each: the source patches
+// of its steps, the steps (with the sentinel's check of the last fields), the
+// records.
+int resident_steps(teuk_solver *s, int n) {
+  for (int done = 0; done < n;) {
+    const int m = std::min(kRing, n - done);
+    ResGate *gates = s->d.ctl->gate;   // (an address on the device)
+    if (s->has_src) HIPCHK(launch_source(s->g, s->d, 0, kRing, true, s->stream));
+    if (s->timing) HIPCHK(timing_begin(s, m * stages_per_step(s->P.integrator)));
+    const int rc = resident_launch(s->stream, [&]() {
+      return launch_resident(s->g, s->d, s->P.integrator, s->has_src, s->res_shape, m, s->nt, gates + s->gate,
+                             wait_ticks(s->res_wait), s->stream);
+    });
+    if (rc) return rc;
+    if (s->timing) HIPCHK(timing_end(s));
+    HIPCHK(launch_finalize(s->g, s->d, m, gates + s->gate, gates + (s->gate ^ 1), s->stream));
+    s->gate ^= 1;
+    s->res_pending = true;
+    done += m;
   }
   return TEUK_OK;
+}
+
+// The control block after everything queued for the solver.  Steps that a
+// resident launch did not take (it could not get all its blocks onto the GPU
+// in time) are run by the per-stage launches first.
+int read_ctl(teuk_solver *s, Ctl &c) {
+  HIPCHK(hipStreamSynchronize(run_stream(s)));
+  HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+  if (c.fail) {
+    const int zero = 0;
+    HIPCHK(hipMemcpy(&s->d.ctl->fail, &zero, sizeof zero, hipMemcpyHostToDevice));
+    s->resident = false;
+    int missing = s->k_host - c.k;
+    while (missing > 0) {
+      const int m = std::min(kRing, missing);
+      const int rc = stage_steps(s, m);
+      if (rc) return rc;
+      missing -= m;
+    }
+    HIPCHK(hipStreamSynchronize(run_stream(s)));
+    HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+  }
+  s->res_pending = false;
+  return TEUK_OK;
+}
+
+// Every queued step is in the solver's memory.
+int settle(teuk_solver *s) {
+  if (!s->res_pending) return TEUK_OK;
+  Ctl c;
+  return read_ctl(s, c);
 }
 
 int build_graph(teuk_solver *s, int steps) {
@@ -187,7 +323,7 @@ int build_graph(teuk_solver *s, int steps) {
   int rc = TEUK_OK;
   for (int i = 0; i < steps && rc == TEUK_OK; i++) rc = enqueue_step(s, i);
   if (rc == TEUK_OK && launch_sentinel(s->g, s->d, s->stream) != hipSuccess) rc = TEUK_EHIP;
-  if (rc == TEUK_OK && launch_finalize(s->g, s->d, steps, s->stream) != hipSuccess) rc = TEUK_EHIP;
+  if (rc == TEUK_OK && launch_finalize(s->g, s->d, steps, nullptr, nullptr, s->stream) != hipSuccess) rc = TEUK_EHIP;
   hipError_t e = hipStreamEndCapture(s->stream, &graph);
   if (rc != TEUK_OK) {
     if (graph) (void)hipGraphDestroy(graph);
@@ -598,6 +734,11 @@ int create_solver(const teuk_params *p, const double *r_h, const double *r_c, co
   }
   if ((g.stag ? launch_init_so2(g, s->d, s->stream) : launch_init_coeffs(g, s->d, s->stream)) != hipSuccess)
     return fail(TEUK_EHIP);
+  // (the exchange counts stages in 32 bits)
+  if (!g.stag && s->nt < (1 << 28) && resident_shape(p->N, p->M, device_cus(), s->res_shape)) {
+    s->resident = true;
+    if (launch_init_res(g, s->d, s->stream) != hipSuccess) return fail(TEUK_EHIP);
+  }
   if (hipStreamSynchronize(s->stream) != hipSuccess) return fail(TEUK_EHIP);
   *out = s;
   return TEUK_OK;
@@ -615,7 +756,10 @@ void teuk_destroy(teuk_solver *s) {
   for (hipEvent_t e : s->ev) (void)hipEventDestroy(e);
   for (void *q : s->allocs) (void)hipFree(q);
   if (s->sched_blk) (void)hipFree(s->sched_blk);
-  if (s->stream) (void)hipStreamDestroy(s->stream);
+  if (s->stream) {
+    chain_forget(s->stream);
+    (void)hipStreamDestroy(s->stream);
+  }
   delete s;
 }
 
@@ -624,6 +768,7 @@ void teuk_destroy(teuk_solver *s) {
 // four real planes q_re, q_im, p_re, p_im (kern.cu:10-13).
 int teuk_set_fields(teuk_solver *s, const double *u) {
   if (!s || !u) return TEUK_EINVAL;
+  if (const int rc = settle(s)) return rc;
   const size_t NM = (size_t)s->P.N * s->P.M;
   std::vector<double> dev(4 * NM);
   for (size_t h = 0; h < 2; h++)
@@ -638,6 +783,7 @@ int teuk_set_fields(teuk_solver *s, const double *u) {
 
 int teuk_get_fields(teuk_solver *s, double *u) {
   if (!s || !u) return TEUK_EINVAL;
+  if (const int rc = settle(s)) return rc;
   const size_t NM = (size_t)s->P.N * s->P.M;
   std::vector<double> dev(4 * NM);
   HIPCHK(hipMemcpyAsync(dev.data(), s->d.U, dev.size() * sizeof(double), hipMemcpyDeviceToHost, run_stream(s)));
@@ -653,6 +799,7 @@ int teuk_get_fields(teuk_solver *s, double *u) {
 int teuk_set_source(teuk_solver *s, const teuk_source_step *steps, int nsteps) {
   if (!s || nsteps < 0) return TEUK_EINVAL;
   if (s->batch) return TEUK_EINVAL;  // the batch's descriptors hold the schedule
+  if (const int rc = settle(s)) return rc;   // steps of the old schedule
   if (!steps || nsteps == 0) {
     // A captured graph holds the source launches and the source-on stage
     // kernels: drop it with the schedule.
@@ -751,16 +898,12 @@ int teuk_step(teuk_solver *s, int nsteps) {
   if (s->k_host + nsteps > s->nt) return TEUK_ERANGE;
   if (s->has_src && s->k_host + nsteps > sched_steps(s)) return TEUK_ERANGE;
   int rc = TEUK_OK;
-  // Direct launches of n steps, closed by one finalize.
-  auto direct = [&](int n) {
-    int r = TEUK_OK;
-    for (int i = 0; i < n && r == TEUK_OK; i++) r = enqueue_step(s, i);
-    if (r == TEUK_OK && n > 0 && launch_sentinel(s->g, s->d, s->stream) != hipSuccess) r = TEUK_EHIP;
-    if (r == TEUK_OK && n > 0 && launch_finalize(s->g, s->d, n, s->stream) != hipSuccess) r = TEUK_EHIP;
-    return r;
-  };
-  if (s->timing) {
-    rc = direct(nsteps);
+  if (s->resident) {
+    rc = resident_steps(s, nsteps);
+  } else if ((rc = settle(s))) {
+    return rc;
+  } else if (s->timing) {
+    rc = stage_steps(s, nsteps);
   } else {
     const int G = 32;
     int left = nsteps;
@@ -771,7 +914,7 @@ int teuk_step(teuk_solver *s, int nsteps) {
         left -= G;
       }
     }
-    if (rc == TEUK_OK) rc = direct(left);
+    if (rc == TEUK_OK) rc = stage_steps(s, left);
   }
   if (rc == TEUK_OK) s->k_host += nsteps;
   return rc;
@@ -779,26 +922,26 @@ int teuk_step(teuk_solver *s, int nsteps) {
 
 int teuk_sync(teuk_solver *s) {
   if (!s) return TEUK_EINVAL;
-  HIPCHK(hipStreamSynchronize(run_stream(s)));
-  if (s->timing) flush_timing(s);
   Ctl c;
-  HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+  const int rc = read_ctl(s, c);
+  if (rc) return rc;
+  if (s->timing) flush_timing(s);
   return c.status ? TEUK_EDIVERGED : TEUK_OK;
 }
 
 int teuk_status(teuk_solver *s) {
   if (!s) return TEUK_EINVAL;
-  HIPCHK(hipStreamSynchronize(run_stream(s)));
   Ctl c;
-  HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+  const int rc = read_ctl(s, c);
+  if (rc) return rc;
   return c.status ? TEUK_EDIVERGED : TEUK_OK;
 }
 
 int teuk_progress(teuk_solver *s, int *k, double *t) {
   if (!s) return TEUK_EINVAL;
   Ctl c;
-  HIPCHK(hipStreamSynchronize(run_stream(s)));
-  HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+  const int rc = read_ctl(s, c);
+  if (rc) return rc;
   if (k) *k = c.k;
   if (t) *t = c.timer;
   return TEUK_OK;
@@ -807,8 +950,8 @@ int teuk_progress(teuk_solver *s, int *k, double *t) {
 int teuk_read_output(teuk_solver *s, int first, int max, teuk_output_row *rows, int *n) {
   if (!s || !rows || first < 0 || max < 0) return TEUK_EINVAL;
   Ctl c;
-  HIPCHK(hipStreamSynchronize(run_stream(s)));
-  HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+  const int rc = read_ctl(s, c);
+  if (rc) return rc;
   const int cnt = std::max(0, std::min(max, c.nrec - first));
   if (cnt > 0) {
     std::vector<double> rec((size_t)cnt * 16);
@@ -830,8 +973,8 @@ int teuk_read_output(teuk_solver *s, int first, int max, teuk_output_row *rows, 
 int teuk_read_psi(teuk_solver *s, int first, int max, double *psi, int *n) {
   if (!s || !psi || first < 0 || max < 0) return TEUK_EINVAL;
   Ctl c;
-  HIPCHK(hipStreamSynchronize(run_stream(s)));
-  HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+  const int rc = read_ctl(s, c);
+  if (rc) return rc;
   const int cnt = std::max(0, std::min(max, c.nrec - first));
   // Each snapshot holds Psi (re, im) followed by the two time integrals.
   // One contiguous copy and a host-side gather: a strided 2D copy into
@@ -962,8 +1105,10 @@ int teuk_set_tiling(teuk_solver *s, int waves_per_block, int waves_per_eu) {
   if (!s || s->batch || s->g.stag) return TEUK_EINVAL;
   if (!(waves_per_block == 1 || waves_per_block == 2 || waves_per_block == 4)) return TEUK_EINVAL;
   if (!(waves_per_eu >= 2 && waves_per_eu <= 4)) return TEUK_EINVAL;
+  if (const int rc = settle(s)) return rc;
   s->tiling.wpb = waves_per_block;
   s->tiling.wpe = waves_per_eu;
+  s->resident = false;
   if (s->gexec) {
     HIPCHK(hipStreamSynchronize(s->stream));
     (void)hipGraphExecDestroy(s->gexec);
@@ -972,10 +1117,25 @@ int teuk_set_tiling(teuk_solver *s, int waves_per_block, int waves_per_eu) {
   return TEUK_OK;
 }
 
+int teuk_set_resident_wait(teuk_solver *s, double seconds) {
+  if (!s || !(seconds >= 0.0)) return TEUK_EINVAL;
+  s->res_wait = seconds;
+  return TEUK_OK;
+}
+
+int teuk_resident(teuk_solver *s, int *on) {
+  if (!s || !on) return TEUK_EINVAL;
+  if (const int rc = settle(s)) return rc;
+  *on = s->resident ? 1 : 0;
+  return TEUK_OK;
+}
+
 int teuk_set_theta_rows(teuk_solver *s, int rows) {
   if (!s || s->batch || s->g.stag) return TEUK_EINVAL;
   if (!theta_rows_ok(s->P.M, rows)) return TEUK_EINVAL;
+  if (const int rc = settle(s)) return rc;
   s->tiling.rows = rows;
+  s->resident = false;
   if (s->gexec) {
     HIPCHK(hipStreamSynchronize(s->stream));
     (void)hipGraphExecDestroy(s->gexec);
@@ -1117,12 +1277,12 @@ int batch_enqueue(teuk_batch *b, const teuk_batch::Group &g, int nsteps) {
   const int nstage = b->integrator == 0 ? 3 : 4;
   for (int k = 0; k < nsteps; k++) {
     if (g.max_cells > 0 && k % kRing == 0)
-      HIPCHK(launch_source_batch(descs, g.count, g.max_cells, k, kRing, b->stream));
+      HIPCHK(launch_source_batch(descs, g.count, g.max_cells, k, kRing, false, b->stream));
     for (int st = 1; st <= nstage; st++)
       HIPCHK(launch_stage_batch(tiles, g.ntiles, b->integrator, st, k, b->tiling, b->stream));
   }
   HIPCHK(launch_sentinel_batch(descs, g.count, b->stream));
-  HIPCHK(launch_finalize_batch(descs, g.count, nsteps, b->stream));
+  HIPCHK(launch_finalize_batch(descs, g.count, nsteps, nullptr, nullptr, b->stream));
   return TEUK_OK;
 }
 
@@ -1268,7 +1428,8 @@ int teuk_batch_sync(teuk_batch *b) {
   int rc = TEUK_OK;
   for (teuk_solver *s : b->members) {
     Ctl c;
-    HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+    const int r = read_ctl(s, c);
+    if (r) return r;
     if (c.status) rc = TEUK_EDIVERGED;
   }
   return rc;
@@ -1310,6 +1471,7 @@ int teuk_source_coeffs(teuk_solver *s, int first, int n, double *c) {
 int teuk_source_patch(teuk_solver *s, int k, double *patch, int *origin) {
   if (!s || !patch || !origin || k < 0) return TEUK_EINVAL;
   if (!s->has_src || k >= s->d.nsched) return TEUK_ERANGE;
+  if (const int rc = settle(s)) return rc;
   hipStream_t st = run_stream(s);
   HIPCHK(hipStreamSynchronize(st));
   HIPCHK(launch_source_at(s->g, s->d, k, st));
@@ -1434,11 +1596,11 @@ int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *th
   for (int done = 0; done < nsteps;) {
     const int n = std::min(kRing, nsteps - done);
     for (int i = 0; i < n; i++) {
-      if (has_src && i == 0) HIPCHK(launch_source(g, d, 0, kRing, st));
+      if (has_src && i == 0) HIPCHK(launch_source(g, d, 0, kRing, false, st));
       for (int s = 1; s <= nstage; s++) HIPCHK(launch_stage(g, d, p->integrator, s, has_src, i, tiling, st));
     }
     HIPCHK(launch_sentinel(g, d, st));
-    HIPCHK(launch_finalize(g, d, n, st));
+    HIPCHK(launch_finalize(g, d, n, nullptr, nullptr, st));
     done += n;
   }
   HIPCHK(hipStreamSynchronize(st));

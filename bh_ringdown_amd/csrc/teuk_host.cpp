@@ -252,4 +252,22 @@ void host_source_prepare(const Grid &g, const SrcStep &st, SrcPrep &out) {
   in.smphi = std::sin(g.m * st.phip);
 }
 
+// The fewest columns per block (a multiple of 8, so that the last block holds
+// at least 8 too: its edge columns and what the rho fill reads) that put the
+// grid on the chip with one block per CU: the narrowest tiles were the fastest
+// at every size (4096x32 RK4: 16 columns 2.9 us a stage, 32 3.0, 64 5.6;
+// 2048x64: 8 columns 3.6, 16 3.5, 32 6.2).  A tile that needs more than eight
+// columns per thread, or more LDS than a CU has, does not fit; nor does a
+// column of more than 64 rows, which must lie within a wave.
+bool resident_shape(int N, int M, int cus, ResShape &sh) {
+  if (M > kWave || M < 16 || M % 8 != 0 || N % 8 != 0 || cus < 1) return false;
+  int C = (((N + cus - 1) / cus) + 7) & ~7;
+  if (C < 8) C = 8;
+  int CP = 1;
+  while (CP < 8 && res_groups(M, CP) * CP < C) CP *= 2;
+  if (res_groups(M, CP) * CP < C || res_lds_bytes(M, C, CP) > kResLdsMax) return false;
+  sh = ResShape{C, (N + C - 1) / C, CP};
+  return true;
+}
+
 }  // namespace teuk

@@ -66,14 +66,25 @@ struct Grid {
                        // its source schedule holds two entries per step
 };
 
+// Gate of a resident launch (teuk_resident.inc): blocks that have arrived,
+// and 0 undecided, 1 the launch runs, 2 it gave up before changing anything.
+// Two per owner, used in turn: the finalize of a launch clears the other one.
+struct ResGate {
+  int arrived;
+  int decision;
+};
+
 // Device control block, one per solver.
 struct Ctl {
   int k;               // completed steps
   int nrec;            // output records written
   int status;          // 0 ok; bit 0: non-finite Psi at the extraction column,
-                       // bit 1: the whole-field sentinel fired (see kGrowthLimit)
-  int pad;
+                       // bit 1: the whole-field sentinel fired (see kGrowthLimit),
+                       // bit 2: a resident launch stopped half way
+  int fail;            // a resident launch gave up: later ones do nothing until
+                       // the host has run the missing steps
   double timer;        // solver time, advanced by repeated addition (body.cu:214)
+  ResGate gate[2];
 };
 
 // Extraction state and output records (device pointers).
@@ -151,6 +162,40 @@ struct BatchTile {
   int pad[3];
 };
 
+// Resident stepping (teuk_resident.inc): B blocks of C rho columns each (the
+// last may hold fewer), CP columns per thread.
+constexpr int kResThreads = 512;
+struct ResShape {
+  int C, B, CP;
+};
+struct ResBlock {
+  int member;          // index into the launch's descriptors
+  int strip, C, B;     // block `strip` of the member's B blocks
+};
+// Column constants the resident kernel reads per stage, [N][8] (subset of kNK).
+enum { kResA, kResBt, kResD, kResC0, kResI0, kResI1, kResBi, kResCi };
+// The set-up plane (DevState::scratch, 8 N M >= 128 N bytes) holds after
+// set-up the exchange flags ([B][32] words, B <= N / 8) and the constants.
+TEUK_HD unsigned *res_flags(const DevState &d) { return reinterpret_cast<unsigned *>(d.scratch); }
+TEUK_HD double *res_k8(const DevState &d, int N) { return d.scratch + 2 * (size_t)N; }
+// LDS of one block: columns of M + 1 rows of two complex fields (C + 8; C + 12
+// for the sweeping kernel of CP >= 4), the extraction integrals, the column
+// constants where they are not scalar loads.
+TEUK_HD constexpr bool res_uniform(int M, int CP) { return CP == 8 && M == kWave; }
+TEUK_HD constexpr size_t res_lds_bytes(int M, int C, int CP) {
+  return (size_t)32 * (C + (CP >= 4 ? 12 : 8)) * (M + 1) + 32 * (size_t)M +
+         (CP >= 4 && !res_uniform(M, CP) ? 64 * (size_t)C : 0);
+}
+// Groups of M threads in a block: any threads for the small-tile kernel,
+// within one wave each for the sweeping one.
+TEUK_HD constexpr int res_groups(int M, int CP) {
+  return CP >= 4 ? (kResThreads / kWave) * (kWave / M) : kResThreads / M;
+}
+constexpr size_t kResLdsMax = 163840 - 512;   // a CU's LDS less the kernel's static part
+// The launch shape for an N x M grid on `cus` CUs, or false if its fields do
+// not fit on the chip.
+bool resident_shape(int N, int M, int cus, ResShape &sh);
+
 // Theta chunks of one rho strip for wavefronts of R rows (R = 2, 4 or 8):
 // the first chunk computes rows 3 .. 2+E and fills rows 0-2 from rows 3 and
 // 4, the last computes rows M-3-E .. M-4 and fills M-3 .. M-1 from M-5 and
@@ -225,12 +270,24 @@ struct Tiling {
 hipError_t launch_init_coeffs(const Grid &g, const DevState &d, hipStream_t s);
 hipError_t launch_source_coeffs(const teuk_t4::StepIn *in, SrcDev *sched, int n, hipStream_t s);
 // Patches of n <= kRing consecutive steps from (step counter + k_rel0).
-hipError_t launch_source(const Grid &g, const DevState &d, int k_rel0, int n, hipStream_t s);
+// colmajor: patches stored column after column (the resident kernel's lanes
+// run along theta), else row after row.
+hipError_t launch_source(const Grid &g, const DevState &d, int k_rel0, int n, bool colmajor, hipStream_t s);
 // The patch of absolute step kstep (into its ring slot).
 hipError_t launch_source_at(const Grid &g, const DevState &d, int kstep, hipStream_t s);
 hipError_t launch_stage(const Grid &g, const DevState &d, int integrator, int stage,
                         bool has_src, int k_rel, Tiling t, hipStream_t s);
-hipError_t launch_finalize(const Grid &g, const DevState &d, int n, hipStream_t s);
+// gate: the gate of the resident launch that ran the steps (the other of its
+// pair is cleared), or null.
+hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, hipStream_t s);
+// Flags and column constants of resident stepping, into the set-up plane.
+hipError_t launch_init_res(const Grid &g, const DevState &d, hipStream_t s);
+// nsteps <= kRing steps of one solve (at most to step nt) in one launch.
+hipError_t launch_resident(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh, int nsteps,
+                           int nt, ResGate *gate, long long limit, hipStream_t s);
+template <int CP>
+hipError_t launch_resident_cp(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh, int nsteps,
+                              int nt, ResGate *gate, long long limit, hipStream_t s);
 // The whole-field sentinel over the current fields (state U); enqueued once
 // per chunk of steps, before the chunk's launch_finalize.
 hipError_t launch_sentinel(const Grid &g, const DevState &d, hipStream_t s);
@@ -241,7 +298,7 @@ hipError_t launch_init_so2(const Grid &g, const DevState &d, hipStream_t s);
 hipError_t launch_so2_step(const Grid &g, const DevState &d, bool has_src, int k_rel, hipStream_t s);
 // Batched forms: one launch covers every member of the batch.
 hipError_t launch_source_batch(const SolveDesc *descs, int nsolves, int max_cells, int k_rel0, int n,
-                               hipStream_t s);
+                               bool colmajor, hipStream_t s);
 hipError_t launch_stage_batch(const BatchTile *tiles, int ntiles, int integrator, int stage, int k_rel, Tiling t,
                               hipStream_t s);
 // The stage builds for R theta rows per wavefront (teuk_stage_r<R>.hip),
@@ -252,7 +309,8 @@ hipError_t launch_stage_rows(const Grid &g, const DevState &d, int integrator, i
 template <int R>
 hipError_t launch_stage_batch_rows(const BatchTile *tiles, int ntiles, int integrator, int stage, int k_rel,
                                    dim3 block, int wpe, hipStream_t s);
-hipError_t launch_finalize_batch(const SolveDesc *descs, int nsolves, int n, hipStream_t s);
+hipError_t launch_finalize_batch(const SolveDesc *descs, int nsolves, int n, ResGate *gate, ResGate *other,
+                                 hipStream_t s);
 // The sentinel of every member still running before the chunk's finalize.
 hipError_t launch_sentinel_batch(const SolveDesc *descs, int nsolves, hipStream_t s);
 // Default launch shape for an N x M grid.

@@ -43,6 +43,18 @@ __global__ __launch_bounds__(256) void k_init_dbdx(Grid g, const double *__restr
 
 
 // ---------------------------------------------------------------------------
+// What resident stepping keeps in the set-up plane once dbdx is formed: its
+// exchange flags, cleared, and the column constants it reads, [N][8].
+__global__ __launch_bounds__(256) void k_init_res(Grid g, DevState d) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= g.N) return;
+  unsigned *flags = res_flags(d);
+  for (int i = 0; i < 4; i++) flags[4 * (size_t)j + i] = 0;
+  constexpr int src[8] = {kKA, kKBt, kKD, kKC0, kKI0, kKI1, kKBi, kKCi};
+#pragma unroll
+  for (int i = 0; i < 8; i++) res_k8(d, g.N)[(size_t)j * 8 + i] = d.ktab[(size_t)src[i] * g.N + j];
+}
+
 // Output records for a batch of n completed steps (body.cu:174-212): for each
 // step k with k % Fr == 0, the energy flux from the snapshot of int Psi dt
 // and the 14 projections of int int Psi dt onto -2Y_lm (proj.c:37-75); the
@@ -50,8 +62,17 @@ __global__ __launch_bounds__(256) void k_init_dbdx(Grid g, const double *__restr
 // round-to-nearest operations in the reference's evaluation order make the
 // records equal the host computation bit for bit.  Then advances the step
 // counter by n.
-__device__ __forceinline__ void finalize_solve(const Grid &g, const Ext &ext_in, Ctl *ctl_in, int n) {
+__device__ __forceinline__ void finalize_solve(const Grid &g, const Ext &ext_in, Ctl *ctl_in, int n,
+                                               const ResGate *gate, ResGate *other) {
   const int M = g.M, t = threadIdx.x;
+  if (gate) {
+    if (t == 0) other->arrived = other->decision = 0;
+    // the launch gave up, or an earlier one had: no step was taken
+    if (gate->decision != 1) {
+      if (t == 0) ctl_in->fail = 1;
+      return;
+    }
+  }
   // global-memory views of the solve's buffers (see global_ptr)
   struct {
     const TEUK_GLOBAL double *snap, *extw, *projw;
@@ -138,15 +159,19 @@ __device__ __forceinline__ void finalize_solve(const Grid &g, const Ext &ext_in,
   }
 }
 
-__global__ __launch_bounds__(256) void k_finalize(Grid g, Ext ext, Ctl *ctl, int n) { finalize_solve(g, ext, ctl, n); }
+__global__ __launch_bounds__(256) void k_finalize(Grid g, Ext ext, Ctl *ctl, int n, const ResGate *gate,
+                                                  ResGate *other) {
+  finalize_solve(g, ext, ctl, n, gate, other);
+}
 
 // One block per solve of the batch; a solve closes at its scheduled step count.
-__global__ __launch_bounds__(256) void k_finalize_batch(const SolveDesc *__restrict__ descs, int n) {
+__global__ __launch_bounds__(256) void k_finalize_batch(const SolveDesc *__restrict__ descs, int n,
+                                                        const ResGate *gate, ResGate *other) {
   const SolveDesc &sd = descs[blockIdx.x];
   const int left = sd.nt - sd.d.ctl->k;
   const int n_eff = n < left ? n : left;
   if (n_eff <= 0) return;
-  finalize_solve(sd.g, sd.d.ext, sd.d.ctl, n_eff);
+  finalize_solve(sd.g, sd.d.ext, sd.d.ctl, n_eff, gate, other);
 }
 
 // Whole-field sentinel (no counterpart in the reference, which checks
@@ -200,6 +225,23 @@ hipError_t launch_init_coeffs(const Grid &g, const DevState &d, hipStream_t s) {
   return hipGetLastError();
 }
 
+hipError_t launch_init_res(const Grid &g, const DevState &d, hipStream_t s) {
+  hipLaunchKernelGGL(k_init_res, dim3((g.N + 255) / 256), dim3(256), 0, s, g, d);
+  return hipGetLastError();
+}
+
+hipError_t launch_resident(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh, int nsteps,
+                           int nt, ResGate *gate, long long limit, hipStream_t s) {
+  if (nsteps < 1 || nsteps > kRing) return hipErrorInvalidValue;
+  switch (sh.CP) {
+    case 1: return launch_resident_cp<1>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
+    case 2: return launch_resident_cp<2>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
+    case 4: return launch_resident_cp<4>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
+    case 8: return launch_resident_cp<8>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 // Launch shape for an N x M grid, from measurements on an MI355X: 2-row
 // wavefronts (2 + (M - 10) / 2 per strip, an odd count, so one wavefront per
 // block), compiled for 3 waves per SIMD from M = 64 up; 4-row wavefronts at
@@ -247,22 +289,24 @@ hipError_t launch_stage_batch(const BatchTile *tiles, int ntiles, int integrator
   }
 }
 
-hipError_t launch_finalize_batch(const SolveDesc *descs, int nsolves, int n, hipStream_t s) {
+hipError_t launch_finalize_batch(const SolveDesc *descs, int nsolves, int n, ResGate *gate, ResGate *other,
+                                 hipStream_t s) {
   if (nsolves <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_finalize_batch, dim3(nsolves), dim3(256), 0, s, descs, n);
+  hipLaunchKernelGGL(k_finalize_batch, dim3(nsolves), dim3(256), 0, s, descs, n, gate, other);
   return hipGetLastError();
 }
 
 hipError_t launch_source_batch(const SolveDesc *descs, int nsolves, int max_cells, int k_rel0, int n,
-                               hipStream_t s) {
+                               bool colmajor, hipStream_t s) {
   if (nsolves <= 0 || max_cells <= 0 || n <= 0) return hipSuccess;
   if (n > kRing) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_source_batch, dim3((max_cells + 255) / 256, nsolves, n), dim3(256), 0, s, descs, k_rel0);
+  hipLaunchKernelGGL(k_source_batch, dim3((max_cells + 255) / 256, nsolves, n), dim3(256), 0, s, descs, k_rel0,
+                     colmajor);
   return hipGetLastError();
 }
 
-hipError_t launch_finalize(const Grid &g, const DevState &d, int n, hipStream_t s) {
-  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, g, d.ext, d.ctl, n);
+hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, hipStream_t s) {
+  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, g, d.ext, d.ctl, n, gate, other);
   return hipGetLastError();
 }
 
@@ -285,11 +329,11 @@ hipError_t launch_sentinel_batch(const SolveDesc *descs, int nsolves, hipStream_
   return hipGetLastError();
 }
 
-hipError_t launch_source(const Grid &g, const DevState &d, int k_rel0, int n, hipStream_t s) {
+hipError_t launch_source(const Grid &g, const DevState &d, int k_rel0, int n, bool colmajor, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   if (n > kRing) return hipErrorInvalidValue;
   const int cells = g.ptsx * g.ptsy;
-  hipLaunchKernelGGL(k_source, dim3((cells + 255) / 256, n), dim3(256), 0, s, g, d, k_rel0);
+  hipLaunchKernelGGL(k_source, dim3((cells + 255) / 256, n), dim3(256), 0, s, g, d, k_rel0, colmajor);
   return hipGetLastError();
 }
 

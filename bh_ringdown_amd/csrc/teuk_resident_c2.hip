@@ -1,0 +1,7 @@
+// Resident stepping with 2 columns per thread (teuk_resident.inc).
+#include "teuk_resident.inc"
+
+namespace teuk {
+template hipError_t launch_resident_cp<2>(const Grid &, const DevState &, int, bool, ResShape, int, int, ResGate *,
+                                          long long, hipStream_t);
+}  // namespace teuk

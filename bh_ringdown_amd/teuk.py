@@ -77,7 +77,7 @@ EXPORTS = [
     "teuk_batch_remove", "teuk_batch_set_tiling", "teuk_batch_step", "teuk_batch_sync", "teuk_batch_info",
     "teuk_source_coeffs", "teuk_source_patch", "teuk_grid_half", "teuk_create_staggered",
     "teuk_trajectory_schedule_staggered", "teuk_status", "teuk_solve_noalloc", "teuk_batch_set_cache_groups",
-    "teuk_ot_transition", "teuk_set_theta_rows", "teuk_batch_set_theta_rows",
+    "teuk_ot_transition", "teuk_set_resident_wait", "teuk_resident", "teuk_set_theta_rows", "teuk_batch_set_theta_rows",
 ]
 
 _lib = None
@@ -131,6 +131,8 @@ def lib():
                                                       ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
         "teuk_set_tiling": ([vp, ctypes.c_int, ctypes.c_int], ctypes.c_int),
         "teuk_set_theta_rows": ([vp, ctypes.c_int], ctypes.c_int),
+        "teuk_resident": ([vp, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
+        "teuk_set_resident_wait": ([vp, ctypes.c_double], ctypes.c_int),
         "teuk_batch_set_theta_rows": ([vp, ctypes.c_int], ctypes.c_int),
         "teuk_ot_transition": ([ctypes.c_double, _dp, _dp], ctypes.c_int),
         "teuk_remaining": ([vp, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
@@ -348,6 +350,16 @@ class Solver:
         _check(lib().teuk_set_tiling(self._h, int(waves_per_block), int(waves_per_eu)), "teuk_set_tiling")
         if theta_rows is not None:
             _check(lib().teuk_set_theta_rows(self._h, int(theta_rows)), "teuk_set_theta_rows")
+
+    def set_resident_wait(self, seconds):
+        """Longest wait of a resident launch for its blocks (teuk_set_resident_wait)."""
+        _check(lib().teuk_set_resident_wait(self._h, float(seconds)), "teuk_set_resident_wait")
+
+    def resident(self):
+        """Whether the next steps keep the fields on the chip (teuk_resident)."""
+        on = ctypes.c_int()
+        _check(lib().teuk_resident(self._h, ctypes.byref(on)), "teuk_resident")
+        return bool(on.value)
 
     def source_coeffs(self, first=0, n=None):
         """Device-computed per-step source coefficients, shape (n, 12)."""

@@ -166,9 +166,9 @@ int teuk_read_output(teuk_solver *s, int first, int max, teuk_output_row *rows, 
 int teuk_read_psi(teuk_solver *s, int first, int max, double *psi, int *n);
 
 /* Kernel timing: when enabled, teuk_step brackets each step's back-to-back
- * stage-kernel launches with a pair of HIP events on the solver stream.
- * teuk_timing returns the number of timed stage launches and their summed
- * duration in milliseconds. */
+ * stage-kernel launches (or each resident launch, of up to 32 steps) with a
+ * pair of HIP events on the solver stream.  teuk_timing returns the number of
+ * timed stages and their summed duration in milliseconds. */
 int teuk_enable_timing(teuk_solver *s, int on);
 int teuk_timing(teuk_solver *s, long long *launches, double *ms);
 
@@ -193,6 +193,18 @@ int teuk_set_tiling(teuk_solver *s, int waves_per_block, int waves_per_eu);
  * rows.  Results do not depend on it.  No counterpart in the reference (its
  * kernels take one thread per point, body.cu:131-165). */
 int teuk_set_theta_rows(teuk_solver *s, int rows);
+
+/* Grids whose fields fit on the chip (M <= 64, up to about a million points)
+ * are stepped with the fields held there, up to 32 steps a launch, until a
+ * launch shape is set for the stage kernels (teuk_set_tiling,
+ * teuk_set_theta_rows).  Such a launch needs all of its blocks on the GPU at
+ * once.  If it does not get them within `seconds` (0.25 by default; 0: it
+ * never waits), because another process holds the CUs, it changes nothing,
+ * and its steps and all later ones are run by the stage kernels.  Results do
+ * not depend on it. */
+int teuk_set_resident_wait(teuk_solver *s, double seconds);
+/* *on: 1 while the solver's next steps would be resident ones, else 0. */
+int teuk_resident(teuk_solver *s, int *on);
 
 /* The 12 per-step source coefficients (the canonical T_4 coefficients times
  * e^{-i m phi_p}/pi, (0,0) (1,0) (0,1) (2,0) (1,1) (0,2) as re, im pairs)

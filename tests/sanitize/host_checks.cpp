@@ -3,8 +3,8 @@
 // g++ -fsanitize=address,undefined and runs it): the grid inversions, the
 // coefficient and projection tables, the source preparation and T4
 // coefficients, the trajectory generator over steep, fast, near-polar and
-// high-spin worldlines, and the stage kernels' theta-chunk layout and block
-// order.  Every output must be finite; any out-of-bounds
+// high-spin worldlines, the stage kernels' theta-chunk layout and block
+// order, and the tiles of resident stepping.  Every output must be finite; any out-of-bounds
 // access or undefined operation aborts the run.
 #include <cmath>
 #include <cstdio>
@@ -149,6 +149,38 @@ void chunk_layout_and_block_order() {
       }
 }
 
+// Tiles of resident stepping: every column in one block, at least 8 in each
+// (edge columns, rho fill), as many threads' columns as the tile has, LDS and
+// the borrowed buffers (exchange slots in the two stage buffers of 4 N M
+// doubles, flags and constants in the set-up plane) large enough.
+void resident_tiles(int cus) {
+  using namespace teuk;
+  for (int M = 8; M <= 128; M += 8)
+    for (int N = 128; N <= 131072; N += (N < 4096 ? 64 : (N < 20000 ? 832 : 4096))) {
+      ResShape sh{0, 0, 0};
+      const bool ok = resident_shape(N, M, cus, sh);
+      if (!ok) {
+        if (M >= 16 && M <= 64 && (long long)N * M <= 400000 && cus >= 256) {
+          std::printf("no resident tile for %dx%d\n", N, M);
+          failures++;
+        }
+        continue;
+      }
+      const int rest = N - (sh.B - 1) * sh.C;
+      const bool sweep = sh.CP >= 4;
+      const size_t xbytes = 2 * (size_t)sh.B * 8 * 32 * M, cbytes = sweep ? 24 * (size_t)N * M : 0;
+      const size_t NM32 = 32 * (size_t)N * M;
+      const bool good = M >= 16 && M <= 64 && sh.B <= cus && sh.C % 8 == 0 && rest >= 8 && rest <= sh.C &&
+                        res_groups(M, sh.CP) >= 8 && res_groups(M, sh.CP) * sh.CP >= sh.C &&
+                        res_lds_bytes(M, sh.C, sh.CP) <= kResLdsMax && xbytes <= (sweep ? NM32 : 2 * NM32) &&
+                        cbytes <= NM32 && 128 * (size_t)sh.B + 64 * (size_t)N <= 8 * (size_t)N * M;
+      if (!good) {
+        std::printf("bad resident tile %dx%d: C %d B %d CP %d\n", N, M, sh.C, sh.B, sh.CP);
+        failures++;
+      }
+    }
+}
+
 }  // namespace
 
 int main() {
@@ -163,6 +195,7 @@ int main() {
   double X, dX;
   for (double L = -40.0; L <= 3.4; L += 0.37)
     if (teuk_ot_transition(L, &X, &dX) != TEUK_OK || !std::isfinite(X) || !std::isfinite(dX)) failures++;
+  for (int cus : {256, 64, 8}) resident_tiles(cus);
   std::printf("host checks: %d failures\n", failures);
   return failures == 0 ? 0 : 1;
 }
