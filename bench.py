@@ -132,7 +132,7 @@ def batch_section(scale, grid=None, plain=True):
     at `scale` of their final time: the plain one-solve-at-a-time loop
     against one batch (plain=False: the batch alone, for profiler runs of
     the batched kernels)."""
-    from bh_ringdown_amd import teuk, tune, workloads
+    from bh_ringdown_amd import teuk, workloads
     items = workloads.batch_72(seed=0, t_final=1200.0 * scale, grid=grid)
     total = sum(p.N * p.M * p.nsteps() for p, _ in items)
     log(f"bench: batch of {len(items)} solves, {total:.3e} point-updates")
@@ -149,14 +149,9 @@ def batch_section(scale, grid=None, plain=True):
     t_plain = time.perf_counter() - t0 if plain else None
     if plain:
         log(f"bench: plain loop {t_plain:.2f} s")
-    shapes = [(p.N, p.M) for p, _ in items]
-    tiling = tune.best_batch_tiling(shapes) or {"waves_per_block": 4, "waves_per_eu": 2, "order": 0, "chunk": 32}
-    groups = tune.best_batch_groups(shapes)
     t0 = time.perf_counter()
     solvers = []
     with teuk.Batch(integrator=1) as b:
-        b.set_tiling(**tiling)
-        b.set_cache_groups(groups)
         for p, rows in items:
             s = teuk.Solver(p)
             s.set_trajectory(rows, p.nsteps())
@@ -175,8 +170,8 @@ def batch_section(scale, grid=None, plain=True):
             "solves_per_hour": 3600.0 * len(items) / t_batch,
             "plain_solves_per_hour": 3600.0 * len(items) / t_plain if plain else None,
             "speedup_vs_plain": t_plain / t_batch if plain else None, "point_updates_per_s": total / t_batch,
-            "plain_point_updates_per_s": total / t_plain if plain else None, "tiling": tiling,
-            "cache_group_bytes": groups, "members_bitwise_equal_alone": same if plain else None}
+            "plain_point_updates_per_s": total / t_plain if plain else None, "tiling": "library default",
+            "members_bitwise_equal_alone": same if plain else None}
 
 
 def serve_section(scale, seconds, policy="sjf"):

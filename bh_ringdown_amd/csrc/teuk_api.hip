@@ -78,12 +78,24 @@ struct teuk_batch {
     int ntiles = 0;
     int max_cells = 0;             // largest source patch of the group (0: no sources)
     hipGraphExec_t gexec = nullptr;
+    // a resident group (teuk_resident.inc): its blocks in d_blocks; CP = 0: stage launches
+    int CP = 0, MT = 0;
+    size_t block_off = 0, lds = 0;
+    int nblocks = 0;
+    double wait = 0.0;
   };
   std::vector<Group> groups;
   SolveDesc *d_desc = nullptr;
   int desc_cap = 0;
   BatchTile *d_tiles = nullptr;
   size_t tiles_cap = 0;
+  // Resident launches for the members whose fields fit on the chip, until a
+  // launch shape is set for the stage kernels.
+  bool resident = true;
+  ResBlock *d_blocks = nullptr;
+  size_t blocks_cap = 0;
+  ResGate *gates = nullptr;        // the pair its resident launches use in turn
+  int gate = 0;
   bool dirty = true;
   int graph_steps = 0;
 };
@@ -292,6 +304,7 @@ int read_ctl(teuk_solver *s, Ctl &c) {
     const int zero = 0;
     HIPCHK(hipMemcpy(&s->d.ctl->fail, &zero, sizeof zero, hipMemcpyHostToDevice));
     s->resident = false;
+    if (s->batch) s->batch->dirty = true;
     int missing = s->k_host - c.k;
     while (missing > 0) {
       const int m = std::min(kRing, missing);
@@ -1170,12 +1183,15 @@ long long member_state_bytes(const teuk_solver *s) {
 // would take the group past group_bytes).
 int batch_rebuild(teuk_batch *b) {
   HIPCHK(hipStreamSynchronize(b->stream));  // kernels may still read the old tables
+  // (a member with steps still to be caught up with would keep its group's gate shut)
+  for (teuk_solver *s : b->members)
+    if (const int rc = settle(s)) return rc;
   batch_drop_graph(b);
   b->groups.clear();
   std::vector<SolveDesc> hd;
   std::vector<BatchTile> table;
-  long long in_group = 0;
-  for (teuk_solver *s : b->members) {
+  std::vector<ResBlock> blocks;
+  auto describe = [b](const teuk_solver *s) {
     SolveDesc sd;
     std::memset(&sd, 0, sizeof sd);
     sd.g = s->g;
@@ -1184,9 +1200,41 @@ int batch_rebuild(teuk_batch *b) {
     sd.ngroups = stage_groups(s->P.M, b->tiling.wpb, b->tiling.rows);
     sd.nt = member_steps(s);
     sd.tiles = (s->P.N / kWave) * sd.ngroups;
-    if (s->k_host >= sd.nt) continue;
+    return sd;
+  };
+  // Resident groups first, then the rest in cache groups.
+  std::vector<teuk_solver *> fit, rest;
+  for (teuk_solver *s : b->members)
+    if (s->k_host < member_steps(s)) (b->resident && s->resident ? fit : rest).push_back(s);
+  std::vector<std::pair<int, int>> shapes;
+  for (teuk_solver *s : fit) shapes.push_back({s->P.N, s->P.M});
+  for (const ResGroup &rg : resident_groups(shapes, device_cus())) {
+    teuk_batch::Group g;
+    g.first = (int)hd.size();
+    g.count = (int)rg.members.size();
+    g.CP = rg.CP;
+    g.MT = rg.MT;
+    g.block_off = blocks.size();
+    g.wait = kResidentWait;
+    for (size_t m = 0; m < rg.members.size(); m++) {
+      teuk_solver *s = fit[rg.members[m]];
+      const int C = rg.C[m];
+      if (s->has_src) g.max_cells = std::max(g.max_cells, s->P.ptsx * s->P.ptsy);
+      g.lds = std::max(g.lds, res_lds_bytes(s->P.M, C, rg.CP));
+      g.wait = std::min(g.wait, s->res_wait);
+      const int B = (s->P.N + C - 1) / C;
+      for (int k = 0; k < B; k++) blocks.push_back(ResBlock{(int)hd.size() - g.first, k, C, B});
+      hd.push_back(describe(s));
+    }
+    g.nblocks = (int)(blocks.size() - g.block_off);
+    b->groups.push_back(g);
+  }
+  const size_t first_stage = b->groups.size();
+  long long in_group = 0;
+  for (teuk_solver *s : rest) {
+    const SolveDesc sd = describe(s);
     const long long sb = member_state_bytes(s);
-    if (b->groups.empty() || (b->group_bytes > 0 && in_group > 0 && in_group + sb > b->group_bytes)) {
+    if (b->groups.size() == first_stage || (b->group_bytes > 0 && in_group > 0 && in_group + sb > b->group_bytes)) {
       teuk_batch::Group g;
       g.first = (int)hd.size();
       b->groups.push_back(g);
@@ -1219,7 +1267,8 @@ int batch_rebuild(teuk_batch *b) {
       return grp == 0 || grp == bt.sd.ngroups - 1;
     });
   };
-  for (auto &g : b->groups) {
+  for (size_t gi = first_stage; gi < b->groups.size(); gi++) {
+    auto &g = b->groups[gi];
     std::vector<BatchTile> list;
     for (int i = 0; i < g.count; i++)
       for (int t = 0; t < hd[g.first + i].tiles; t++) {
@@ -1261,6 +1310,15 @@ int batch_rebuild(teuk_batch *b) {
       return TEUK_ENOMEM;
     b->tiles_cap = std::max<size_t>(table.size(), 1);
   }
+  if (blocks.size() > b->blocks_cap) {
+    if (b->d_blocks) (void)hipFree(b->d_blocks);
+    b->d_blocks = nullptr;
+    b->blocks_cap = 0;
+    if (hipMalloc(&b->d_blocks, blocks.size() * sizeof(ResBlock)) != hipSuccess) return TEUK_ENOMEM;
+    b->blocks_cap = blocks.size();
+  }
+  if (!blocks.empty())
+    HIPCHK(hipMemcpy(b->d_blocks, blocks.data(), blocks.size() * sizeof(ResBlock), hipMemcpyHostToDevice));
   if (n > 0) HIPCHK(hipMemcpy(b->d_desc, hd.data(), (size_t)n * sizeof(SolveDesc), hipMemcpyHostToDevice));
   if (!table.empty())
     HIPCHK(hipMemcpy(b->d_tiles, table.data(), table.size() * sizeof(BatchTile), hipMemcpyHostToDevice));
@@ -1283,6 +1341,25 @@ int batch_enqueue(teuk_batch *b, const teuk_batch::Group &g, int nsteps) {
   }
   HIPCHK(launch_sentinel_batch(descs, g.count, b->stream));
   HIPCHK(launch_finalize_batch(descs, g.count, nsteps, nullptr, nullptr, b->stream));
+  return TEUK_OK;
+}
+
+// The same by resident launches of up to kRing steps.
+int batch_resident(teuk_batch *b, const teuk_batch::Group &g, int nsteps) {
+  const SolveDesc *descs = b->d_desc + g.first;
+  for (int done = 0; done < nsteps;) {
+    const int m = std::min(kRing, nsteps - done);
+    if (g.max_cells > 0) HIPCHK(launch_source_batch(descs, g.count, g.max_cells, 0, kRing, true, b->stream));
+    ResGate *gate = b->gates + b->gate, *other = b->gates + (b->gate ^ 1);
+    const int rc = resident_launch(b->stream, [&]() {
+      return launch_resident_batch(descs, b->d_blocks + g.block_off, g.nblocks, b->integrator, g.CP, g.MT, g.lds, m,
+                                   gate, wait_ticks(g.wait), b->stream);
+    });
+    if (rc) return rc;
+    HIPCHK(launch_finalize_batch(descs, g.count, m, gate, other, b->stream));
+    b->gate ^= 1;
+    done += m;
+  }
   return TEUK_OK;
 }
 
@@ -1320,6 +1397,11 @@ int teuk_batch_create(int integrator, long long hbm_budget, teuk_batch **out) {
     delete b;
     return TEUK_EHIP;
   }
+  if (hipMalloc(&b->gates, 2 * sizeof(ResGate)) != hipSuccess ||
+      hipMemset(b->gates, 0, 2 * sizeof(ResGate)) != hipSuccess) {
+    teuk_batch_destroy(b);
+    return TEUK_ENOMEM;
+  }
   *out = b;
   return TEUK_OK;
 }
@@ -1331,6 +1413,9 @@ void teuk_batch_destroy(teuk_batch *b) {
   batch_drop_graph(b);
   if (b->d_desc) (void)hipFree(b->d_desc);
   if (b->d_tiles) (void)hipFree(b->d_tiles);
+  if (b->d_blocks) (void)hipFree(b->d_blocks);
+  if (b->gates) (void)hipFree(b->gates);
+  chain_forget(b->stream);
   (void)hipStreamDestroy(b->stream);
   delete b;
 }
@@ -1344,6 +1429,7 @@ int teuk_batch_set_tiling(teuk_batch *b, int waves_per_block, int waves_per_eu, 
   b->tiling.wpe = waves_per_eu;
   b->order = order;
   b->chunk = chunk;
+  b->resident = false;
   b->dirty = true;
   return TEUK_OK;
 }
@@ -1351,6 +1437,7 @@ int teuk_batch_set_tiling(teuk_batch *b, int waves_per_block, int waves_per_eu, 
 int teuk_batch_set_theta_rows(teuk_batch *b, int rows) {
   if (!b || !(rows == 2 || rows == 4 || rows == 8)) return TEUK_EINVAL;
   b->tiling.rows = rows;
+  b->resident = false;
   b->dirty = true;
   return TEUK_OK;
 }
@@ -1400,7 +1487,10 @@ int teuk_batch_step(teuk_batch *b, int nsteps) {
     // cache through its chunk)
     const int n = std::min(left, b->chunk);
     for (auto &g : b->groups) {
-      if (n == b->chunk) {
+      if (g.CP) {
+        const int rc = batch_resident(b, g, n);
+        if (rc) return rc;
+      } else if (n == b->chunk) {
         if (!g.gexec || b->graph_steps != b->chunk) {
           int rc = batch_build_graph(b, g);
           if (rc) return rc;
@@ -1415,6 +1505,7 @@ int teuk_batch_step(teuk_batch *b, int nsteps) {
       const int nt = member_steps(s);
       const int before = s->k_host;
       s->k_host = std::min(nt, s->k_host + n);
+      s->res_pending = true;
       if (before < nt && s->k_host >= nt) b->dirty = true;  // drop its tiles next chunk
     }
     left -= n;

@@ -1,6 +1,7 @@
 // Host-side set-up for libteuk: the compactified grid with its Newton
 // inversion r(r*), the -2Y_lm projection weights and the trajectory
 // consumption pattern of the reference driver.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -265,9 +266,94 @@ bool resident_shape(int N, int M, int cus, ResShape &sh) {
   if (C < 8) C = 8;
   int CP = 1;
   while (CP < 8 && res_groups(M, CP) * CP < C) CP *= 2;
-  if (res_groups(M, CP) * CP < C || res_lds_bytes(M, C, CP) > kResLdsMax) return false;
+  if (res_groups(M, CP) * CP < C || res_lds_bytes(M, C, CP) > kResLdsMax || C < res_least_tile(M, CP)) return false;
   sh = ResShape{C, (N + C - 1) / C, CP};
   return true;
+}
+
+// The widest tile of CP columns per thread (0: none).
+static int widest_tile(int M, int CP) {
+  int C = (res_groups(M, CP) * CP) & ~7;
+  while (C >= 8 && res_lds_bytes(M, C, CP) > kResLdsMax) C -= 8;
+  return C >= res_least_tile(M, CP) ? C : 0;
+}
+
+// A launch takes as long as its tiles, whatever they belong to, so members
+// share launches, and wide tiles put more of them into one: a stage takes
+// about 2.8, 3.1, 5.4, 8.8 us with tiles of 1, 2, 4, 8 columns per thread and
+// up to 32 rows, 3.3, 3.8, 6.0, 10.4 us with up to 64 (MI355X).  For the
+// members of each row class (32, 64, others) the tile width with the least
+// sum over its launches is taken, the launches filled in order of size, and
+// each launch's tiles then narrowed as far as the CUs allow.
+std::vector<ResGroup> resident_groups(const std::vector<std::pair<int, int>> &shapes, int cus) {
+  static const int kCP[4] = {1, 2, 4, 8};
+  static const double kStage32[4] = {2.8, 3.1, 5.4, 8.8}, kStage64[4] = {3.3, 3.8, 6.0, 10.4};
+  std::vector<ResGroup> out;
+  for (int cls : {32, 64, 0}) {
+    std::vector<int> own;
+    bool tall = false;
+    for (size_t i = 0; i < shapes.size(); i++) {
+      const int M = shapes[i].second;
+      ResShape sh;
+      if ((M == 32 || M == 64 ? M : 0) != cls || !resident_shape(shapes[i].first, M, cus, sh)) continue;
+      own.push_back((int)i);
+      tall = tall || M > 32;
+    }
+    std::stable_sort(own.begin(), own.end(), [&](int x, int y) {
+      return (long long)shapes[x].first * shapes[x].second > (long long)shapes[y].first * shapes[y].second;
+    });
+    // a member's tile of about `want` columns, and its blocks
+    auto tile = [&](int i, int CP, int want) {
+      const int M = shapes[i].second;
+      return std::min(widest_tile(M, CP), std::max(want, res_least_tile(M, CP)));
+    };
+    auto blocks = [&](int i, int CP, int want) {
+      const int C = tile(i, CP, want);
+      return C ? (shapes[i].first + C - 1) / C : cus + 1;
+    };
+    auto total = [&](const std::vector<int> &m, int CP, int want) {
+      long long nb = 0;
+      for (int i : m) nb += blocks(i, CP, want);
+      return nb;
+    };
+    const int kWide = 1 << 20;
+    std::vector<std::vector<int>> best;
+    double best_cost = 0.0;
+    for (int c = 0; c < 4 && !own.empty(); c++) {
+      std::vector<std::vector<int>> bins;
+      std::vector<int> used;
+      for (int i : own) {
+        const int nb = blocks(i, kCP[c], kWide);
+        size_t k = 0;
+        while (k < bins.size() && used[k] + nb > cus) k++;
+        if (k == bins.size()) {
+          bins.push_back({});
+          used.push_back(0);
+        }
+        bins[k].push_back(i);
+        used[k] += nb;
+      }
+      const bool fits = *std::max_element(used.begin(), used.end()) <= cus;
+      const double cost = (double)bins.size() * (tall ? kStage64 : kStage32)[c];
+      if (fits && (best.empty() || cost < best_cost)) {
+        best = bins;
+        best_cost = cost;
+      }
+    }
+    for (std::vector<int> &m : best) {
+      ResGroup g;
+      g.CP = 8;
+      for (int c = 3; c >= 0; c--)
+        if (total(m, kCP[c], kWide) <= cus) g.CP = kCP[c];
+      int want = 8;
+      while (total(m, g.CP, want) > cus) want += 8;
+      for (int i : m) g.C.push_back(tile(i, g.CP, want));
+      g.members = std::move(m);
+      g.MT = g.CP >= 4 ? cls : 0;
+      out.push_back(g);
+    }
+  }
+  return out;
 }
 
 }  // namespace teuk

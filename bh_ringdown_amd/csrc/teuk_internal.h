@@ -6,6 +6,8 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <utility>
+#include <vector>
 
 #define TEUK_HD __host__ __device__ inline
 #include "teuk_point.h"
@@ -186,15 +188,31 @@ TEUK_HD constexpr size_t res_lds_bytes(int M, int C, int CP) {
   return (size_t)32 * (C + (CP >= 4 ? 12 : 8)) * (M + 1) + 32 * (size_t)M +
          (CP >= 4 && !res_uniform(M, CP) ? 64 * (size_t)C : 0);
 }
+// The row count a kernel of CP columns per thread is built for (0: any).
+TEUK_HD constexpr int res_built_rows(int M, int CP) { return CP >= 4 && (M == 64 || M == 32) ? M : 0; }
 // Groups of M threads in a block: any threads for the small-tile kernel,
 // within one wave each for the sweeping one.
 TEUK_HD constexpr int res_groups(int M, int CP) {
   return CP >= 4 ? (kResThreads / kWave) * (kWave / M) : kResThreads / M;
 }
+// The narrowest tile: a sweep reads the halo on its far side in its second
+// phase, so no column of the first may reach it.
+TEUK_HD constexpr int res_least_tile(int M, int CP) { return CP >= 4 ? res_groups(M, CP) * (CP / 2) + 8 : 8; }
 constexpr size_t kResLdsMax = 163840 - 512;   // a CU's LDS less the kernel's static part
 // The launch shape for an N x M grid on `cus` CUs, or false if its fields do
 // not fit on the chip.
 bool resident_shape(int N, int M, int cus, ResShape &sh);
+
+// Members of a batch that run in one resident launch: their tiles take at
+// most one block per CU.
+struct ResGroup {
+  std::vector<int> members;   // indices into the shapes given
+  std::vector<int> C;         // tile width of each
+  int CP, MT;                 // columns per thread, the built-in M (0: any)
+};
+// The launches for members of the given N x M on `cus` CUs; a member whose
+// fields do not fit on the chip is in none.
+std::vector<ResGroup> resident_groups(const std::vector<std::pair<int, int>> &shapes, int cus);
 
 // Theta chunks of one rho strip for wavefronts of R rows (R = 2, 4 or 8):
 // the first chunk computes rows 3 .. 2+E and fills rows 0-2 from rows 3 and
@@ -285,6 +303,13 @@ hipError_t launch_init_res(const Grid &g, const DevState &d, hipStream_t s);
 // nsteps <= kRing steps of one solve (at most to step nt) in one launch.
 hipError_t launch_resident(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh, int nsteps,
                            int nt, ResGate *gate, long long limit, hipStream_t s);
+// The same for the blocks of several solves (a group of resident_groups), each
+// at most to its own last step; lds: the largest member's res_lds_bytes.
+hipError_t launch_resident_batch(const SolveDesc *descs, const ResBlock *blocks, int nblocks, int integrator, int CP,
+                                 int MT, size_t lds, int nsteps, ResGate *gate, long long limit, hipStream_t s);
+template <int CP>
+hipError_t launch_resident_batch_cp(const SolveDesc *descs, const ResBlock *blocks, int nblocks, int integrator, int MT,
+                                    size_t lds, int nsteps, ResGate *gate, long long limit, hipStream_t s);
 template <int CP>
 hipError_t launch_resident_cp(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh, int nsteps,
                               int nt, ResGate *gate, long long limit, hipStream_t s);

@@ -170,6 +170,7 @@ __global__ __launch_bounds__(256) void k_finalize_batch(const SolveDesc *__restr
   const SolveDesc &sd = descs[blockIdx.x];
   const int left = sd.nt - sd.d.ctl->k;
   const int n_eff = n < left ? n : left;
+  if (gate && blockIdx.x == 0 && threadIdx.x == 0) other->arrived = other->decision = 0;
   if (n_eff <= 0) return;
   finalize_solve(sd.g, sd.d.ext, sd.d.ctl, n_eff, gate, other);
 }
@@ -238,6 +239,18 @@ hipError_t launch_resident(const Grid &g, const DevState &d, int integrator, boo
     case 2: return launch_resident_cp<2>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
     case 4: return launch_resident_cp<4>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
     case 8: return launch_resident_cp<8>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_resident_batch(const SolveDesc *descs, const ResBlock *blocks, int nblocks, int integrator, int CP,
+                                 int MT, size_t lds, int nsteps, ResGate *gate, long long limit, hipStream_t s) {
+  if (nblocks < 1 || nsteps < 1 || nsteps > kRing || lds > kResLdsMax) return hipErrorInvalidValue;
+  switch (CP) {
+    case 1: return launch_resident_batch_cp<1>(descs, blocks, nblocks, integrator, MT, lds, nsteps, gate, limit, s);
+    case 2: return launch_resident_batch_cp<2>(descs, blocks, nblocks, integrator, MT, lds, nsteps, gate, limit, s);
+    case 4: return launch_resident_batch_cp<4>(descs, blocks, nblocks, integrator, MT, lds, nsteps, gate, limit, s);
+    case 8: return launch_resident_batch_cp<8>(descs, blocks, nblocks, integrator, MT, lds, nsteps, gate, limit, s);
     default: return hipErrorInvalidValue;
   }
 }

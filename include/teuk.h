@@ -226,9 +226,12 @@ int teuk_remaining(teuk_solver *s, int *steps);
 /* ---- batches ------------------------------------------------------------------ */
 /* No counterpart in the reference (body() solves one mode per call; the
  * reference runs modes and trajectories as separate jobs, main.c:50-55,
- * run.sh:3-16).  A batch steps many solvers together: each RK stage of every
- * member is one launch (blocks index a table of {solver, tile}); chunks of
- * steps are captured in a hipGraph.  Members may differ in N, M, a, m, dt,
+ * run.sh:3-16).  A batch steps many solvers together.  Members whose fields
+ * fit on the chip share resident launches (teuk_set_resident_wait), as many
+ * to a launch as the CUs hold, until a launch shape is set for the batch
+ * (teuk_batch_set_tiling, teuk_batch_set_theta_rows).  For the others each RK
+ * stage of every member is one launch (blocks index a table of {solver,
+ * tile}); chunks of steps are captured in a hipGraph.  Members may differ in N, M, a, m, dt,
  * source and length; each stops at its own schedule end.  A member's results
  * are bitwise those of stepping it alone.  Members must share the
  * integrator.  While in a batch a solver is stepped only by its batch;

@@ -170,7 +170,7 @@ void resident_tiles(int cus) {
       const bool sweep = sh.CP >= 4;
       const size_t xbytes = 2 * (size_t)sh.B * 8 * 32 * M, cbytes = sweep ? 24 * (size_t)N * M : 0;
       const size_t NM32 = 32 * (size_t)N * M;
-      const bool good = M >= 16 && M <= 64 && sh.B <= cus && sh.C % 8 == 0 && rest >= 8 && rest <= sh.C &&
+      const bool good = M >= 16 && M <= 64 && sh.B <= cus && sh.C % 8 == 0 && sh.C >= res_least_tile(M, sh.CP) && rest >= 8 && rest <= sh.C &&
                         res_groups(M, sh.CP) >= 8 && res_groups(M, sh.CP) * sh.CP >= sh.C &&
                         res_lds_bytes(M, sh.C, sh.CP) <= kResLdsMax && xbytes <= (sweep ? NM32 : 2 * NM32) &&
                         cbytes <= NM32 && 128 * (size_t)sh.B + 64 * (size_t)N <= 8 * (size_t)N * M;
@@ -179,6 +179,42 @@ void resident_tiles(int cus) {
         failures++;
       }
     }
+}
+
+// Launches of a batch: every member that fits on the chip in exactly one, at
+// most one block per CU, a tile that its kernel takes for every member.
+void resident_batches(int cus) {
+  using namespace teuk;
+  unsigned long long rng = 12345;
+  auto next = [&](int n) { rng = rng * 6364136223846793005ULL + 1442695040888963407ULL; return (int)((rng >> 33) % n); };
+  static const int kM[] = {16, 24, 32, 40, 48, 56, 64, 72};
+  for (int trial = 0; trial < 300; trial++) {
+    std::vector<std::pair<int, int>> shapes;
+    const int n = next(24), same = next(3) == 0 ? 8 * (2 + next(8)) : 0;
+    for (int i = 0; i < n; i++) shapes.push_back({64 * (2 + next(next(2) ? 300 : 60)), same ? same : kM[next(8)]});
+    std::vector<int> seen(n, 0);
+    bool good = true;
+    for (const ResGroup &g : resident_groups(shapes, cus)) {
+      int nb = 0;
+      for (size_t m = 0; m < g.members.size(); m++) {
+        const int i = g.members[m], C = g.C[m], N = shapes[i].first, M = shapes[i].second;
+        const int rest = N - ((N + C - 1) / C - 1) * C;
+        seen[i]++;
+        nb += (N + C - 1) / C;
+        good = good && C >= res_least_tile(M, g.CP) && C % 8 == 0 && rest >= 8 && res_groups(M, g.CP) * g.CP >= C &&
+               res_lds_bytes(M, C, g.CP) <= kResLdsMax && g.MT == res_built_rows(M, g.CP);
+      }
+      good = good && nb <= cus && !g.members.empty();
+    }
+    for (int i = 0; i < n; i++) {
+      ResShape sh;
+      good = good && seen[i] == (resident_shape(shapes[i].first, shapes[i].second, cus, sh) ? 1 : 0);
+    }
+    if (!good) {
+      std::printf("bad resident launches for a batch of %d (trial %d, %d CUs)\n", n, trial, cus);
+      failures++;
+    }
+  }
 }
 
 }  // namespace
@@ -195,7 +231,10 @@ int main() {
   double X, dX;
   for (double L = -40.0; L <= 3.4; L += 0.37)
     if (teuk_ot_transition(L, &X, &dX) != TEUK_OK || !std::isfinite(X) || !std::isfinite(dX)) failures++;
-  for (int cus : {256, 64, 8}) resident_tiles(cus);
+  for (int cus : {256, 64, 8}) {
+    resident_tiles(cus);
+    resident_batches(cus);
+  }
   std::printf("host checks: %d failures\n", failures);
   return failures == 0 ? 0 : 1;
 }

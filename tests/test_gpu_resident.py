@@ -157,3 +157,42 @@ def test_resident_solvers_on_several_threads():
         t.join()
     for i in range(len(specs)):
         assert np.array_equal(got[i][0], ref[i]) and got[i][1], i
+
+
+BATCH = [  # N, M, m, steps, source: several row classes, narrow and wide tiles, one that does not fit
+    (256, 16, 2, 40, True), (4096, 32, 2, 40, True), (8192, 32, -3, 33, False), (4096, 32, 0, 64, True),
+    (16384, 32, 1, 20, False), (8192, 64, 2, 40, True), (2048, 64, 3, 12, False), (6080, 40, 2, 40, True),
+    (1024, 24, -1, 70, False), (512, 72, 2, 40, True),
+]
+
+
+@pytest.mark.parametrize("integrator,wait", [(1, None), (0, None), (1, 0.0)])
+def test_batch_of_resident_members_equal_alone(integrator, wait):
+    """Members of one batch in shared resident launches, each as alone; with
+    a wait of zero for one member its launch gives up and its members' steps
+    are caught up with by the stage kernels."""
+    specs = [setup(N, M, integrator, m, steps, N // 2 + 5, src, seed=i) for i, (N, M, m, steps, src) in enumerate(BATCH)]
+    ref = []
+    for (p, u0, rows), c in zip(specs, BATCH):
+        with start(p, u0, rows, c[3]) as s:
+            s.step(c[3])
+            s.sync()
+            ref.append((s.get_fields(), s.output(), s.psi()))
+    solvers = [start(p, u0, rows, c[3]) for (p, u0, rows), c in zip(specs, BATCH)]
+    if wait is not None:
+        solvers[1].set_resident_wait(wait)
+    with teuk.Batch(integrator=integrator) as b:
+        for s in solvers:
+            assert b.add(s)
+        b.step(13)
+        b.step(35)
+        b.step(70)
+        b.sync()
+        assert b.info()["active"] == 0
+        for s, (u, out, psi), c in zip(solvers, ref, BATCH):
+            assert s.progress()[0] == c[3], c
+            assert np.array_equal(s.get_fields(), u) and np.array_equal(s.psi(), psi), c
+            o = s.output()
+            assert np.array_equal(o["h"], out["h"]) and np.array_equal(o["t"], out["t"]), c
+    for s in solvers:
+        s.close()
