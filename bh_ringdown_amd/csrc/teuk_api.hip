@@ -153,11 +153,18 @@ struct ResidentChain {
 constexpr int kMaxDevices = 64;
 ResidentChain g_chain[kMaxDevices];
 
+// The current device's chain.
+ResidentChain *resident_chain() {
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+  return &g_chain[dev];
+}
+
 template <class Launch>
 int resident_launch(hipStream_t stream, Launch launch) {
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return TEUK_EHIP;
-  ResidentChain &c = g_chain[dev];
+  ResidentChain *chain = resident_chain();
+  if (!chain) return TEUK_EHIP;
+  ResidentChain &c = *chain;
   std::lock_guard<std::mutex> hold(c.lock);
   if (!c.done) HIPCHK(hipEventCreateWithFlags(&c.done, hipEventDisableTiming));
   if (c.last && c.last != stream) HIPCHK(hipStreamWaitEvent(stream, c.done, 0));
@@ -1679,24 +1686,50 @@ int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *th
     HIPCHK(launch_source_coeffs(reinterpret_cast<const teuk_t4::StepIn *>(base + off_sched + b_dev), d.sched,
                                 nsteps, st));
   }
-  // the steps, in the launch sequence of teuk_step: chunks of kRing steps
-  // (patches for the chunk, the fused stages of each step), each closed by
-  // the sentinel and the output records
+  // the steps, in the launch sequences of teuk_step: chunks of kRing steps
+  // (patches for the chunk, then one resident launch or the fused stages of
+  // each step with the sentinel), each closed by the output records
   const Tiling tiling = default_tiling(p->N, p->M);
   const int nstage = stages_per_step(p->integrator);
-  for (int done = 0; done < nsteps;) {
-    const int n = std::min(kRing, nsteps - done);
-    for (int i = 0; i < n; i++) {
-      if (has_src && i == 0) HIPCHK(launch_source(g, d, 0, kRing, false, st));
-      for (int s = 1; s <= nstage; s++) HIPCHK(launch_stage(g, d, p->integrator, s, has_src, i, tiling, st));
+  auto stage_chunks = [&](int left) {
+    for (; left > 0; left -= kRing) {
+      const int n = std::min(kRing, left);
+      for (int i = 0; i < n; i++) {
+        if (has_src && i == 0) HIPCHK(launch_source(g, d, 0, kRing, false, st));
+        for (int s = 1; s <= nstage; s++) HIPCHK(launch_stage(g, d, p->integrator, s, has_src, i, tiling, st));
+      }
+      HIPCHK(launch_sentinel(g, d, st));
+      HIPCHK(launch_finalize(g, d, n, nullptr, nullptr, st));
     }
-    HIPCHK(launch_sentinel(g, d, st));
-    HIPCHK(launch_finalize(g, d, n, nullptr, nullptr, st));
-    done += n;
+    return TEUK_OK;
+  };
+  ResShape sh{0, 0, 0};
+  Ctl c;
+  if (nsteps < (1 << 28) && resident_shape(p->N, p->M, device_cus(), sh)) {
+    // This solve's place in the chain of resident launches is held until its
+    // last one has ended: that takes no event.
+    ResidentChain *chain = resident_chain();
+    if (!chain) return TEUK_EHIP;
+    std::lock_guard<std::mutex> turn(chain->lock);
+    if (chain->last) HIPCHK(hipStreamWaitEvent(st, chain->done, 0));
+    HIPCHK(launch_init_res(g, d, st));
+    int gate = 0;
+    for (int done = 0; done < nsteps; done += kRing, gate ^= 1) {
+      const int n = std::min(kRing, nsteps - done);
+      if (has_src) HIPCHK(launch_source(g, d, 0, kRing, true, st));
+      HIPCHK(launch_resident(g, d, p->integrator, has_src, sh, n, nsteps, d.ctl->gate + gate,
+                             wait_ticks(kResidentWait), st));
+      HIPCHK(launch_finalize(g, d, n, d.ctl->gate + gate, d.ctl->gate + (gate ^ 1), st));
+    }
+    HIPCHK(hipStreamSynchronize(st));
+    chain->last = nullptr;   // (waited for above)
+    HIPCHK(hipMemcpy(&c, d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+    if (c.fail && (rc = stage_chunks(nsteps - c.k))) return rc;
+  } else if ((rc = stage_chunks(nsteps))) {
+    return rc;
   }
   HIPCHK(hipStreamSynchronize(st));
   // results back (teuk_get_fields, teuk_read_output)
-  Ctl c;
   HIPCHK(hipMemcpy(&c, d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
   if (u_out) {
     const double *dev = reinterpret_cast<const double *>(stage);
