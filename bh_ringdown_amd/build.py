@@ -24,7 +24,8 @@ HIPFLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contrac
 
 # The stage kernels are built once per theta-chunk length, one object each
 # (the longest compiles first).
-LIB_SOURCES = ["teuk_resident_c8.hip", "teuk_resident_c4.hip", "teuk_resident_c2.hip", "teuk_resident_c1.hip",
+LIB_SOURCES = ["teuk_resident_c8.hip", "teuk_resident_c6.hip", "teuk_resident_c4.hip", "teuk_resident_c2.hip",
+               "teuk_resident_c1.hip",
                "teuk_stage_r8.hip", "teuk_stage_r4.hip", "teuk_stage_r2.hip", "teuk_kernels.hip", "teuk_so2.hip",
                "teuk_api.hip", "teuk_host.cpp", "teuk_traj.cpp"]
 

@@ -36,6 +36,15 @@ struct teuk_solver {
   double res_wait = kResidentWait;
   int gate = 0;                  // which of the control block's two gates is next
   bool res_pending = false;      // resident launches since the control block was last read
+  // Grids beyond the chip: stepped in segments (resident_segments), from the
+  // state U into D, which then change places.  The places at the start of
+  // each chunk since the control block was last read, by step.
+  ResSegments segs;
+  struct Place {
+    int k;
+    double *U, *D;
+  };
+  std::vector<Place> places;
   teuk_batch *batch = nullptr;   // set while a batch drives this solver
   hipStream_t stream = nullptr;
   int nt = 0;              // scheduled steps: (int)(T/dt), body.cu:59
@@ -282,18 +291,48 @@ int stage_steps(teuk_solver *s, int n) {
 // of its steps, the steps (with the sentinel's check of the last fields), the
 // records.
 int resident_steps(teuk_solver *s, int n) {
+  const bool whole = s->segs.spans.empty();
+  const int most = whole ? kRing : s->segs.steps;
   for (int done = 0; done < n;) {
-    const int m = std::min(kRing, n - done);
-    ResGate *gates = s->d.ctl->gate;   // (an address on the device)
-    if (s->has_src) HIPCHK(launch_source(s->g, s->d, 0, kRing, true, s->stream));
+    const int m = std::min(most, n - done);
+    // (addresses on the device)
+    const int sets = whole ? 1 : kMaxSegments;
+    ResGate *gates = whole ? s->d.ctl->gate : res_gates(s->d, s->P.N);
+    ResGate *mine = gates + s->gate * sets, *other = gates + (s->gate ^ 1) * sets;
+    if (s->has_src) HIPCHK(launch_source(s->g, s->d, 0, m, true, s->stream));
     if (s->timing) HIPCHK(timing_begin(s, m * stages_per_step(s->P.integrator)));
-    const int rc = resident_launch(s->stream, [&]() {
-      return launch_resident(s->g, s->d, s->P.integrator, s->has_src, s->res_shape, m, s->nt, gates + s->gate,
-                             wait_ticks(s->res_wait), s->stream);
-    });
+    auto launch = [&](const ResShape &sh, const ResSpan &sp, ResGate *gate) {
+      return resident_launch(s->stream, [&]() {
+        return launch_resident(s->g, s->d, s->P.integrator, s->has_src, sh, sp, m, s->nt, gate,
+                               wait_ticks(s->res_wait), s->stream);
+      });
+    };
+    int rc = TEUK_OK;
+    int used = 1;
+    if (whole) {
+      rc = launch(s->res_shape, ResSpan{0, s->P.N, 0, s->P.N, s->d.U, s->d.D, nullptr, 0}, mine);
+    } else {
+      // The segment with the extraction column goes last: its time integrals
+      // are in place, and must not have moved if another launch gives up.
+      s->places.push_back({s->k_host + done, s->d.U, s->d.D});
+      used = (int)s->segs.spans.size();
+      std::vector<ResSpan> order = s->segs.spans;
+      std::stable_partition(order.begin(), order.end(),
+                            [&](const ResSpan &sp) { return s->g.je < sp.v0 || s->g.je >= sp.v1; });
+      for (int i = 0; i < used && rc == TEUK_OK; i++) {
+        ResSpan sp = order[i];
+        ResShape sh = s->segs.sh;
+        sh.B = (sp.s1 - sp.s0 + sh.C - 1) / sh.C;
+        sp.out = s->d.D;
+        sp.cpl = s->d.C + (size_t)sh.B * 64 * s->P.M;   // behind the exchange slots
+        sp.prev = i ? mine + i - 1 : nullptr;
+        rc = launch(sh, sp, mine + i);
+      }
+    }
     if (rc) return rc;
     if (s->timing) HIPCHK(timing_end(s));
-    HIPCHK(launch_finalize(s->g, s->d, m, gates + s->gate, gates + (s->gate ^ 1), s->stream));
+    HIPCHK(launch_finalize(s->g, s->d, m, mine + used - 1, other, s->stream, used));
+    if (!whole) std::swap(s->d.U, s->d.D);
     s->gate ^= 1;
     s->res_pending = true;
     done += m;
@@ -311,6 +350,12 @@ int read_ctl(teuk_solver *s, Ctl &c) {
     const int zero = 0;
     HIPCHK(hipMemcpy(&s->d.ctl->fail, &zero, sizeof zero, hipMemcpyHostToDevice));
     s->resident = false;
+    for (const teuk_solver::Place &p : s->places)
+      if (p.k == c.k) {   // where the first launch that gave up left the state
+        s->d.U = p.U;
+        s->d.D = p.D;
+        break;
+      }
     if (s->batch) s->batch->dirty = true;
     int missing = s->k_host - c.k;
     while (missing > 0) {
@@ -323,6 +368,7 @@ int read_ctl(teuk_solver *s, Ctl &c) {
     HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
   }
   s->res_pending = false;
+  s->places.clear();
   return TEUK_OK;
 }
 
@@ -755,9 +801,13 @@ int create_solver(const teuk_params *p, const double *r_h, const double *r_c, co
   if ((g.stag ? launch_init_so2(g, s->d, s->stream) : launch_init_coeffs(g, s->d, s->stream)) != hipSuccess)
     return fail(TEUK_EHIP);
   // (the exchange counts stages in 32 bits)
-  if (!g.stag && s->nt < (1 << 28) && resident_shape(p->N, p->M, device_cus(), s->res_shape)) {
-    s->resident = true;
-    if (launch_init_res(g, s->d, s->stream) != hipSuccess) return fail(TEUK_EHIP);
+  if (!g.stag && s->nt < (1 << 28)) {
+    s->resident = resident_shape(p->N, p->M, device_cus(), s->res_shape);
+    if (!s->resident) {
+      s->segs = resident_segments(p->N, p->M, p->integrator, device_cus());
+      s->resident = !s->segs.spans.empty();
+    }
+    if (s->resident && launch_init_res(g, s->d, s->stream) != hipSuccess) return fail(TEUK_EHIP);
   }
   if (hipStreamSynchronize(s->stream) != hipSuccess) return fail(TEUK_EHIP);
   *out = s;
@@ -1212,7 +1262,8 @@ int batch_rebuild(teuk_batch *b) {
   // Resident groups first, then the rest in cache groups.
   std::vector<teuk_solver *> fit, rest;
   for (teuk_solver *s : b->members)
-    if (s->k_host < member_steps(s)) (b->resident && s->resident ? fit : rest).push_back(s);
+    if (s->k_host < member_steps(s))
+      (b->resident && s->resident && s->segs.spans.empty() ? fit : rest).push_back(s);
   std::vector<std::pair<int, int>> shapes;
   for (teuk_solver *s : fit) shapes.push_back({s->P.N, s->P.M});
   for (const ResGroup &rg : resident_groups(shapes, device_cus())) {
@@ -1356,7 +1407,7 @@ int batch_resident(teuk_batch *b, const teuk_batch::Group &g, int nsteps) {
   const SolveDesc *descs = b->d_desc + g.first;
   for (int done = 0; done < nsteps;) {
     const int m = std::min(kRing, nsteps - done);
-    if (g.max_cells > 0) HIPCHK(launch_source_batch(descs, g.count, g.max_cells, 0, kRing, true, b->stream));
+    if (g.max_cells > 0) HIPCHK(launch_source_batch(descs, g.count, g.max_cells, 0, m, true, b->stream));
     ResGate *gate = b->gates + b->gate, *other = b->gates + (b->gate ^ 1);
     const int rc = resident_launch(b->stream, [&]() {
       return launch_resident_batch(descs, b->d_blocks + g.block_off, g.nblocks, b->integrator, g.CP, g.MT, g.lds, m,
@@ -1716,9 +1767,9 @@ int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *th
     int gate = 0;
     for (int done = 0; done < nsteps; done += kRing, gate ^= 1) {
       const int n = std::min(kRing, nsteps - done);
-      if (has_src) HIPCHK(launch_source(g, d, 0, kRing, true, st));
-      HIPCHK(launch_resident(g, d, p->integrator, has_src, sh, n, nsteps, d.ctl->gate + gate,
-                             wait_ticks(kResidentWait), st));
+      if (has_src) HIPCHK(launch_source(g, d, 0, n, true, st));
+      HIPCHK(launch_resident(g, d, p->integrator, has_src, sh, ResSpan{0, p->N, 0, p->N, d.U, d.D, nullptr, 0}, n, nsteps,
+                             d.ctl->gate + gate, wait_ticks(kResidentWait), st));
       HIPCHK(launch_finalize(g, d, n, d.ctl->gate + gate, d.ctl->gate + (gate ^ 1), st));
     }
     HIPCHK(hipStreamSynchronize(st));

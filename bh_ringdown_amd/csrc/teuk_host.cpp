@@ -259,16 +259,23 @@ void host_source_prepare(const Grid &g, const SrcStep &st, SrcPrep &out) {
 // at every size (4096x32 RK4: 16 columns 2.9 us a stage, 32 3.0, 64 5.6;
 // 2048x64: 8 columns 3.6, 16 3.5, 32 6.2).  A tile that needs more than eight
 // columns per thread, or more LDS than a CU has, does not fit; nor does a
-// column of more than 64 rows, which must lie within a wave.
+// column of more than 128 rows, which must lie within two waves.
 bool resident_shape(int N, int M, int cus, ResShape &sh) {
-  if (M > kWave || M < 16 || M % 8 != 0 || N % 8 != 0 || cus < 1) return false;
-  int C = (((N + cus - 1) / cus) + 7) & ~7;
-  if (C < 8) C = 8;
-  int CP = 1;
-  while (CP < 8 && res_groups(M, CP) * CP < C) CP *= 2;
-  if (res_groups(M, CP) * CP < C || res_lds_bytes(M, C, CP) > kResLdsMax || C < res_least_tile(M, CP)) return false;
-  sh = ResShape{C, (N + C - 1) / C, CP};
-  return true;
+  if (M > 2 * kWave || M < 16 || M % 8 != 0 || N % 8 != 0 || cus < 1) return false;
+  const int fit = std::max(8, (((N + cus - 1) / cus) + 7) & ~7);
+  for (int CP : kResCP) {
+    const int C = std::max(fit, res_least_tile(M, CP));
+    if (res_groups(M, CP) * CP < C || res_lds_bytes(M, C, CP) > kResLdsMax) continue;
+    sh = ResShape{C, (N + C - 1) / C, CP};
+    return true;
+  }
+  return false;
+}
+
+// Measured time of one stage with tiles of kResCP[c] columns per thread (us).
+static double stage_us(int M, int c) {
+  static const double k32[5] = {2.8, 3.1, 5.4, 7.2, 8.8}, k64[5] = {3.3, 3.8, 6.0, 8.2, 10.4};
+  return M <= 32 ? k32[c] : k64[c];
 }
 
 // The widest tile of CP columns per thread (0: none).
@@ -279,25 +286,22 @@ static int widest_tile(int M, int CP) {
 }
 
 // A launch takes as long as its tiles, whatever they belong to, so members
-// share launches, and wide tiles put more of them into one: a stage takes
-// about 2.8, 3.1, 5.4, 8.8 us with tiles of 1, 2, 4, 8 columns per thread and
-// up to 32 rows, 3.3, 3.8, 6.0, 10.4 us with up to 64 (MI355X).  For the
-// members of each row class (32, 64, others) the tile width with the least
-// sum over its launches is taken, the launches filled in order of size, and
-// each launch's tiles then narrowed as far as the CUs allow.
+// share launches, and wide tiles put more of them into one.  For the members
+// of each row class (the row counts kernels are built for, others together)
+// the tile width with the least sum of stage_us over its launches is taken,
+// the launches filled in order of size, and each launch's tiles then narrowed
+// as far as the CUs allow.
 std::vector<ResGroup> resident_groups(const std::vector<std::pair<int, int>> &shapes, int cus) {
-  static const int kCP[4] = {1, 2, 4, 8};
-  static const double kStage32[4] = {2.8, 3.1, 5.4, 8.8}, kStage64[4] = {3.3, 3.8, 6.0, 10.4};
   std::vector<ResGroup> out;
-  for (int cls : {32, 64, 0}) {
+  for (int cls : {32, 64, 128, kAnyTall, 0}) {
     std::vector<int> own;
-    bool tall = false;
+    int tallest = 0;
     for (size_t i = 0; i < shapes.size(); i++) {
       const int M = shapes[i].second;
       ResShape sh;
-      if ((M == 32 || M == 64 ? M : 0) != cls || !resident_shape(shapes[i].first, M, cus, sh)) continue;
+      if (res_built_rows(M, 8) != cls || !resident_shape(shapes[i].first, M, cus, sh)) continue;
       own.push_back((int)i);
-      tall = tall || M > 32;
+      tallest = std::max(tallest, M);
     }
     std::stable_sort(own.begin(), own.end(), [&](int x, int y) {
       return (long long)shapes[x].first * shapes[x].second > (long long)shapes[y].first * shapes[y].second;
@@ -319,11 +323,11 @@ std::vector<ResGroup> resident_groups(const std::vector<std::pair<int, int>> &sh
     const int kWide = 1 << 20;
     std::vector<std::vector<int>> best;
     double best_cost = 0.0;
-    for (int c = 0; c < 4 && !own.empty(); c++) {
+    for (int c = 0; c < 5 && !own.empty(); c++) {
       std::vector<std::vector<int>> bins;
       std::vector<int> used;
       for (int i : own) {
-        const int nb = blocks(i, kCP[c], kWide);
+        const int nb = blocks(i, kResCP[c], kWide);
         size_t k = 0;
         while (k < bins.size() && used[k] + nb > cus) k++;
         if (k == bins.size()) {
@@ -334,7 +338,7 @@ std::vector<ResGroup> resident_groups(const std::vector<std::pair<int, int>> &sh
         used[k] += nb;
       }
       const bool fits = *std::max_element(used.begin(), used.end()) <= cus;
-      const double cost = (double)bins.size() * (tall ? kStage64 : kStage32)[c];
+      const double cost = (double)bins.size() * stage_us(tallest, c);
       if (fits && (best.empty() || cost < best_cost)) {
         best = bins;
         best_cost = cost;
@@ -343,8 +347,8 @@ std::vector<ResGroup> resident_groups(const std::vector<std::pair<int, int>> &sh
     for (std::vector<int> &m : best) {
       ResGroup g;
       g.CP = 8;
-      for (int c = 3; c >= 0; c--)
-        if (total(m, kCP[c], kWide) <= cus) g.CP = kCP[c];
+      for (int c = 4; c >= 0; c--)
+        if (total(m, kResCP[c], kWide) <= cus) g.CP = kResCP[c];
       int want = 8;
       while (total(m, g.CP, want) > cus) want += 8;
       for (int i : m) g.C.push_back(tile(i, g.CP, want));
@@ -354,6 +358,53 @@ std::vector<ResGroup> resident_groups(const std::vector<std::pair<int, int>> &sh
     }
   }
   return out;
+}
+
+// Tiles of each width and 4 to 32 steps a launch: the segments cover the
+// columns beside them that the steps reach (H on each inner side), so fewer
+// steps mean less to compute twice and more launches, each about 25 us of
+// loads, stores and set-up.  The per-stage kernels take about 19.5 us a stage
+// and million points; the plan must beat that by a tenth.
+ResSegments resident_segments(int N, int M, int integrator, int cus) {
+  ResSegments best;
+  ResShape whole;
+  if (M > 2 * kWave || M < 16 || M % 8 != 0 || N % 8 != 0 || cus < 1 || resident_shape(N, M, cus, whole)) return best;
+  const int S = integrator == 0 ? 3 : 4;
+  double best_cost = 0.9 * S * 19.5e-6 * (double)N * M;
+  for (int c = 2; c < 5; c++) {
+    const int C = widest_tile(M, kResCP[c]);
+    for (int steps = 4; C && steps <= kRing; steps *= 2) {
+      const int cap = C * cus, H = 4 * S * steps;
+      if (cap <= 2 * H) continue;
+      int k = 2;
+      while (2LL * (cap - H) + (long long)(k - 2) * (cap - 2 * H) < N) k++;
+      const double cost = k * (S * stage_us(M, c) + 25.0 / steps);
+      if (k > kMaxSegments || cost >= best_cost) continue;
+      const int w = ((N - 2 * H + k - 1) / k + 7) & ~7;   // an inner segment's own columns; the outer ones' are H more
+      ResSegments r;
+      r.steps = steps;
+      bool good = w >= 8;
+      int widest = 0;
+      for (int i = 0, v0 = 0; i < k && good; i++) {
+        const int v1 = i == k - 1 ? N : std::min(N, v0 + w + (i == 0 ? H : 0));
+        ResSpan sp{std::max(0, v0 - H), std::min(N, v1 + H), v0, v1, nullptr, nullptr, nullptr, 0};
+        widest = std::max(widest, sp.s1 - sp.s0);
+        good = v1 > v0 && sp.s1 - sp.s0 <= cap;
+        r.spans.push_back(sp);
+        v0 = v1;
+      }
+      const int Cn = std::max(res_least_tile(M, kResCP[c]), (((widest + cus - 1) / cus) + 7) & ~7);
+      r.sh = ResShape{Cn, (widest + Cn - 1) / Cn, kResCP[c]};
+      for (int i = 0; i < k && good; i++) r.spans[i].flag_blk = i * r.sh.B;
+      // the stage buffer that holds exchange slots and coefficient values; the flags' place
+      good = good && Cn <= C && 512LL * r.sh.B + 24LL * widest <= 32LL * N &&
+             128LL * k * r.sh.B + 16 * kMaxSegments <= 16LL * N;
+      if (!good) continue;
+      best = r;
+      best_cost = cost;
+    }
+  }
+  return best;
 }
 
 }  // namespace teuk

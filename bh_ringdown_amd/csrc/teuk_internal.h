@@ -174,34 +174,66 @@ struct ResBlock {
   int member;          // index into the launch's descriptors
   int strip, C, B;     // block `strip` of the member's B blocks
 };
+// The columns [s0, s1) of a launch, those of them it stores ([v0, v1), into
+// `out`), its plane for the coefficient values, the launch before it in the
+// same steps (or null) and its first block's flags.
+struct ResSpan {
+  int s0, s1, v0, v1;
+  double *out, *cpl;
+  const ResGate *prev;
+  int flag_blk;
+};
 // Column constants the resident kernel reads per stage, [N][8] (subset of kNK).
 enum { kResA, kResBt, kResD, kResC0, kResI0, kResI1, kResBi, kResCi };
 // The set-up plane (DevState::scratch, 8 N M >= 128 N bytes) holds after
-// set-up the exchange flags ([B][32] words, B <= N / 8) and the constants.
+// set-up the exchange flags ([blocks][32] words), the gates of segments' launches
+// ([2][kMaxSegments], at the end of 16 N bytes) and the constants.
+constexpr int kMaxSegments = 32;
 TEUK_HD unsigned *res_flags(const DevState &d) { return reinterpret_cast<unsigned *>(d.scratch); }
+TEUK_HD ResGate *res_gates(const DevState &d, int N) {
+  return reinterpret_cast<ResGate *>(d.scratch + 2 * (size_t)N) - 2 * kMaxSegments;
+}
 TEUK_HD double *res_k8(const DevState &d, int N) { return d.scratch + 2 * (size_t)N; }
+// The row count a kernel of CP columns per thread is built for: 0 any up to
+// 64, kAnyTall any of 65 to 128 (two waves a column).
+constexpr int kAnyTall = 1;
+TEUK_HD constexpr int res_built_rows(int M, int CP) {
+  if (CP < 4) return 0;
+  return M == 128 || M == 64 || M == 32 ? M : (M > kWave ? kAnyTall : 0);
+}
+// Groups of M threads in a block: any threads for the small-tile kernel (at
+// least 8, one per edge column), within one or two waves each for the sweeping one.
+TEUK_HD constexpr int res_groups(int M, int CP) {
+  return CP >= 4 ? (M > kWave ? 4 : (kResThreads / kWave) * (kWave / M)) : (M > kWave ? 0 : kResThreads / M);
+}
 // LDS of one block: columns of M + 1 rows of two complex fields (C + 8; C + 12
 // for the sweeping kernel of CP >= 4), the extraction integrals, the column
 // constants where they are not scalar loads.
-TEUK_HD constexpr bool res_uniform(int M, int CP) { return CP == 8 && M == kWave; }
+TEUK_HD constexpr bool res_uniform(int M, int CP) { return CP > 4 && M >= kWave; }
 TEUK_HD constexpr size_t res_lds_bytes(int M, int C, int CP) {
   return (size_t)32 * (C + (CP >= 4 ? 12 : 8)) * (M + 1) + 32 * (size_t)M +
          (CP >= 4 && !res_uniform(M, CP) ? 64 * (size_t)C : 0);
 }
-// The row count a kernel of CP columns per thread is built for (0: any).
-TEUK_HD constexpr int res_built_rows(int M, int CP) { return CP >= 4 && (M == 64 || M == 32) ? M : 0; }
-// Groups of M threads in a block: any threads for the small-tile kernel,
-// within one wave each for the sweeping one.
-TEUK_HD constexpr int res_groups(int M, int CP) {
-  return CP >= 4 ? (kResThreads / kWave) * (kWave / M) : kResThreads / M;
-}
 // The narrowest tile: a sweep reads the halo on its far side in its second
 // phase, so no column of the first may reach it.
-TEUK_HD constexpr int res_least_tile(int M, int CP) { return CP >= 4 ? res_groups(M, CP) * (CP / 2) + 8 : 8; }
+TEUK_HD constexpr int res_least_tile(int M, int CP) { return CP >= 4 ? ((res_groups(M, CP) * (CP / 2) + 11) & ~7) : 8; }
 constexpr size_t kResLdsMax = 163840 - 512;   // a CU's LDS less the kernel's static part
+constexpr int kResCP[5] = {1, 2, 4, 6, 8};
 // The launch shape for an N x M grid on `cus` CUs, or false if its fields do
 // not fit on the chip.
 bool resident_shape(int N, int M, int cus, ResShape &sh);
+
+// A grid that does not fit is stepped in segments of its columns, `steps`
+// steps of one after the other: a segment's launch also computes the columns
+// beside it that its steps reach (4 per stage), so segments need nothing from
+// each other, and stores its own into a second state.  Empty: the per-stage
+// kernels are faster, or the solve's buffers are too small for it.
+struct ResSegments {
+  int steps = 0;
+  ResShape sh{0, 0, 0};             // of every segment (B: the widest)
+  std::vector<ResSpan> spans;       // s0 .. v1 and flag_blk
+};
+ResSegments resident_segments(int N, int M, int integrator, int cus);
 
 // Members of a batch that run in one resident launch: their tiles take at
 // most one block per CU.
@@ -296,13 +328,14 @@ hipError_t launch_source_at(const Grid &g, const DevState &d, int kstep, hipStre
 hipError_t launch_stage(const Grid &g, const DevState &d, int integrator, int stage,
                         bool has_src, int k_rel, Tiling t, hipStream_t s);
 // gate: the gate of the resident launch that ran the steps (the other of its
-// pair is cleared), or null.
-hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, hipStream_t s);
+// pair, or all `others` of it, is cleared), or null.
+hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, hipStream_t s,
+                           int others = 1);
 // Flags and column constants of resident stepping, into the set-up plane.
 hipError_t launch_init_res(const Grid &g, const DevState &d, hipStream_t s);
 // nsteps <= kRing steps of one solve (at most to step nt) in one launch.
-hipError_t launch_resident(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh, int nsteps,
-                           int nt, ResGate *gate, long long limit, hipStream_t s);
+hipError_t launch_resident(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh,
+                           const ResSpan &sp, int nsteps, int nt, ResGate *gate, long long limit, hipStream_t s);
 // The same for the blocks of several solves (a group of resident_groups), each
 // at most to its own last step; lds: the largest member's res_lds_bytes.
 hipError_t launch_resident_batch(const SolveDesc *descs, const ResBlock *blocks, int nblocks, int integrator, int CP,
@@ -311,8 +344,8 @@ template <int CP>
 hipError_t launch_resident_batch_cp(const SolveDesc *descs, const ResBlock *blocks, int nblocks, int integrator, int MT,
                                     size_t lds, int nsteps, ResGate *gate, long long limit, hipStream_t s);
 template <int CP>
-hipError_t launch_resident_cp(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh, int nsteps,
-                              int nt, ResGate *gate, long long limit, hipStream_t s);
+hipError_t launch_resident_cp(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh,
+                              const ResSpan &sp, int nsteps, int nt, ResGate *gate, long long limit, hipStream_t s);
 // The whole-field sentinel over the current fields (state U); enqueued once
 // per chunk of steps, before the chunk's launch_finalize.
 hipError_t launch_sentinel(const Grid &g, const DevState &d, hipStream_t s);

@@ -63,10 +63,10 @@ __global__ __launch_bounds__(256) void k_init_res(Grid g, DevState d) {
 // records equal the host computation bit for bit.  Then advances the step
 // counter by n.
 __device__ __forceinline__ void finalize_solve(const Grid &g, const Ext &ext_in, Ctl *ctl_in, int n,
-                                               const ResGate *gate, ResGate *other) {
+                                               const ResGate *gate, ResGate *other, int others = 1) {
   const int M = g.M, t = threadIdx.x;
   if (gate) {
-    if (t == 0) other->arrived = other->decision = 0;
+    if (t < others) other[t].arrived = other[t].decision = 0;
     // the launch gave up, or an earlier one had: no step was taken
     if (gate->decision != 1) {
       if (t == 0) ctl_in->fail = 1;
@@ -160,8 +160,8 @@ __device__ __forceinline__ void finalize_solve(const Grid &g, const Ext &ext_in,
 }
 
 __global__ __launch_bounds__(256) void k_finalize(Grid g, Ext ext, Ctl *ctl, int n, const ResGate *gate,
-                                                  ResGate *other) {
-  finalize_solve(g, ext, ctl, n, gate, other);
+                                                  ResGate *other, int others) {
+  finalize_solve(g, ext, ctl, n, gate, other, others);
 }
 
 // One block per solve of the batch; a solve closes at its scheduled step count.
@@ -231,14 +231,17 @@ hipError_t launch_init_res(const Grid &g, const DevState &d, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_resident(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh, int nsteps,
-                           int nt, ResGate *gate, long long limit, hipStream_t s) {
-  if (nsteps < 1 || nsteps > kRing) return hipErrorInvalidValue;
+hipError_t launch_resident(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh,
+                           const ResSpan &sp, int nsteps, int nt, ResGate *gate, long long limit, hipStream_t s) {
+  if (nsteps < 1 || nsteps > kRing || sp.s0 + (long long)sh.B * sh.C < sp.s1 ||
+      sp.s1 - sp.s0 - (long long)(sh.B - 1) * sh.C < 8)
+    return hipErrorInvalidValue;
   switch (sh.CP) {
-    case 1: return launch_resident_cp<1>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
-    case 2: return launch_resident_cp<2>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
-    case 4: return launch_resident_cp<4>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
-    case 8: return launch_resident_cp<8>(g, d, integrator, has_src, sh, nsteps, nt, gate, limit, s);
+    case 1: return launch_resident_cp<1>(g, d, integrator, has_src, sh, sp, nsteps, nt, gate, limit, s);
+    case 2: return launch_resident_cp<2>(g, d, integrator, has_src, sh, sp, nsteps, nt, gate, limit, s);
+    case 4: return launch_resident_cp<4>(g, d, integrator, has_src, sh, sp, nsteps, nt, gate, limit, s);
+    case 6: return launch_resident_cp<6>(g, d, integrator, has_src, sh, sp, nsteps, nt, gate, limit, s);
+    case 8: return launch_resident_cp<8>(g, d, integrator, has_src, sh, sp, nsteps, nt, gate, limit, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -250,6 +253,7 @@ hipError_t launch_resident_batch(const SolveDesc *descs, const ResBlock *blocks,
     case 1: return launch_resident_batch_cp<1>(descs, blocks, nblocks, integrator, MT, lds, nsteps, gate, limit, s);
     case 2: return launch_resident_batch_cp<2>(descs, blocks, nblocks, integrator, MT, lds, nsteps, gate, limit, s);
     case 4: return launch_resident_batch_cp<4>(descs, blocks, nblocks, integrator, MT, lds, nsteps, gate, limit, s);
+    case 6: return launch_resident_batch_cp<6>(descs, blocks, nblocks, integrator, MT, lds, nsteps, gate, limit, s);
     case 8: return launch_resident_batch_cp<8>(descs, blocks, nblocks, integrator, MT, lds, nsteps, gate, limit, s);
     default: return hipErrorInvalidValue;
   }
@@ -318,8 +322,9 @@ hipError_t launch_source_batch(const SolveDesc *descs, int nsolves, int max_cell
   return hipGetLastError();
 }
 
-hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, hipStream_t s) {
-  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, g, d.ext, d.ctl, n, gate, other);
+hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, hipStream_t s,
+                           int others) {
+  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, g, d.ext, d.ctl, n, gate, other, others);
   return hipGetLastError();
 }
 

@@ -2,8 +2,8 @@
 #include "teuk_resident.inc"
 
 namespace teuk {
-template hipError_t launch_resident_cp<1>(const Grid &, const DevState &, int, bool, ResShape, int, int, ResGate *,
-                                          long long, hipStream_t);
+template hipError_t launch_resident_cp<1>(const Grid &, const DevState &, int, bool, ResShape, const ResSpan &, int, int,
+                                          ResGate *, long long, hipStream_t);
 template hipError_t launch_resident_batch_cp<1>(const SolveDesc *, const ResBlock *, int, int, int, size_t, int, ResGate *,
                                                 long long, hipStream_t);
 }  // namespace teuk

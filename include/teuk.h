@@ -194,11 +194,12 @@ int teuk_set_tiling(teuk_solver *s, int waves_per_block, int waves_per_eu);
  * kernels take one thread per point, body.cu:131-165). */
 int teuk_set_theta_rows(teuk_solver *s, int rows);
 
-/* Grids whose fields fit on the chip (M <= 64, up to about a million points)
- * are stepped with the fields held there, up to 32 steps a launch, until a
- * launch shape is set for the stage kernels (teuk_set_tiling,
- * teuk_set_theta_rows).  Such a launch needs all of its blocks on the GPU at
- * once.  If it does not get them within `seconds` (0.25 by default; 0: it
+/* Grids of up to 128 theta rows are stepped with their fields held on the
+ * chip, up to 32 steps a launch, until a launch shape is set for the stage
+ * kernels (teuk_set_tiling, teuk_set_theta_rows): grids of up to about a
+ * million points whole, larger ones in segments of rho columns, one after
+ * the other, where that is faster.  Such a launch needs all of its blocks on
+ * the GPU at once.  If it does not get them within `seconds` (0.25 by default; 0: it
  * never waits), because another process holds the CUs, it changes nothing,
  * and its steps and all later ones are run by the stage kernels.  Results do
  * not depend on it. */

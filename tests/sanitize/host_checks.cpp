@@ -155,7 +155,7 @@ void chunk_layout_and_block_order() {
 // doubles, flags and constants in the set-up plane) large enough.
 void resident_tiles(int cus) {
   using namespace teuk;
-  for (int M = 8; M <= 128; M += 8)
+  for (int M = 8; M <= 136; M += 8)
     for (int N = 128; N <= 131072; N += (N < 4096 ? 64 : (N < 20000 ? 832 : 4096))) {
       ResShape sh{0, 0, 0};
       const bool ok = resident_shape(N, M, cus, sh);
@@ -170,8 +170,8 @@ void resident_tiles(int cus) {
       const bool sweep = sh.CP >= 4;
       const size_t xbytes = 2 * (size_t)sh.B * 8 * 32 * M, cbytes = sweep ? 24 * (size_t)N * M : 0;
       const size_t NM32 = 32 * (size_t)N * M;
-      const bool good = M >= 16 && M <= 64 && sh.B <= cus && sh.C % 8 == 0 && sh.C >= res_least_tile(M, sh.CP) && rest >= 8 && rest <= sh.C &&
-                        res_groups(M, sh.CP) >= 8 && res_groups(M, sh.CP) * sh.CP >= sh.C &&
+      const bool good = M >= 16 && M <= 128 && sh.B <= cus && sh.C % 8 == 0 && sh.C >= res_least_tile(M, sh.CP) && rest >= 8 && rest <= sh.C &&
+                        res_groups(M, sh.CP) >= (sweep ? 4 : 8) && res_groups(M, sh.CP) * sh.CP >= sh.C &&
                         res_lds_bytes(M, sh.C, sh.CP) <= kResLdsMax && xbytes <= (sweep ? NM32 : 2 * NM32) &&
                         cbytes <= NM32 && 128 * (size_t)sh.B + 64 * (size_t)N <= 8 * (size_t)N * M;
       if (!good) {
@@ -181,13 +181,50 @@ void resident_tiles(int cus) {
     }
 }
 
+// Segments of grids beyond the chip: their own columns tile the grid, each
+// launch reaches as far beside them as its steps do (or to the grid's edge),
+// is one that its kernel takes, and finds room in the borrowed buffers.
+void resident_spans(int cus) {
+  using namespace teuk;
+  int planned = 0;
+  for (int M = 8; M <= 136; M += 8)
+    for (int N = 1024; N <= 131072; N += (N < 20000 ? 1600 : 5824))
+      for (int integ = 0; integ < 2; integ++) {
+        const ResSegments r = resident_segments(N, M, integ, cus);
+        if (r.spans.empty()) continue;
+        planned++;
+        const int H = 4 * (integ ? 4 : 3) * r.steps, C = r.sh.C, CP = r.sh.CP, k = (int)r.spans.size();
+        bool good = M >= 16 && M <= 128 && r.steps >= 1 && r.steps <= kRing && k >= 2 && k <= kMaxSegments &&
+                    r.sh.B <= cus && C % 8 == 0 && C >= res_least_tile(M, CP) && res_groups(M, CP) * CP >= C &&
+                    res_lds_bytes(M, C, CP) <= kResLdsMax;
+        int at = 0;
+        for (int i = 0; i < k; i++) {
+          const ResSpan &sp = r.spans[i];
+          const int len = sp.s1 - sp.s0, B = (len + C - 1) / C;
+          good = good && sp.v0 == at && sp.v1 > sp.v0 && sp.s0 == (sp.v0 > H ? sp.v0 - H : 0) &&
+                 sp.s1 == (sp.v1 + H < N ? sp.v1 + H : N) && B <= r.sh.B && len - (B - 1) * C >= 8 && len % 8 == 0 &&
+                 sp.flag_blk >= i * r.sh.B && 512LL * B * M + 24LL * len * M <= 32LL * N * M &&
+                 128LL * (sp.flag_blk + B) + 16 * kMaxSegments <= 16LL * N;
+          at = sp.v1;
+        }
+        if (!good || at != N) {
+          std::printf("bad segments for %dx%d integrator %d on %d CUs\n", N, M, integ, cus);
+          failures++;
+        }
+      }
+  if (cus == 256 && planned < 20) {
+    std::printf("only %d grids in segments\n", planned);
+    failures++;
+  }
+}
+
 // Launches of a batch: every member that fits on the chip in exactly one, at
 // most one block per CU, a tile that its kernel takes for every member.
 void resident_batches(int cus) {
   using namespace teuk;
   unsigned long long rng = 12345;
   auto next = [&](int n) { rng = rng * 6364136223846793005ULL + 1442695040888963407ULL; return (int)((rng >> 33) % n); };
-  static const int kM[] = {16, 24, 32, 40, 48, 56, 64, 72};
+  static const int kM[] = {16, 24, 32, 40, 48, 64, 72, 128};
   for (int trial = 0; trial < 300; trial++) {
     std::vector<std::pair<int, int>> shapes;
     const int n = next(24), same = next(3) == 0 ? 8 * (2 + next(8)) : 0;
@@ -233,6 +270,7 @@ int main() {
     if (teuk_ot_transition(L, &X, &dX) != TEUK_OK || !std::isfinite(X) || !std::isfinite(dX)) failures++;
   for (int cus : {256, 64, 8}) {
     resident_tiles(cus);
+    resident_spans(cus);
     resident_batches(cus);
   }
   std::printf("host checks: %d failures\n", failures);

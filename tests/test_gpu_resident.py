@@ -68,6 +68,17 @@ CASES = [  # N, M, integrator, m, steps, extraction column, source
     (16384, 64, 1, 2, 33, 4160, True),    # sweeps, four columns a phase, scalar column constants
     (16000, 64, 0, 3, 12, 15999, True),
     (32768, 32, 1, 2, 8, 8191, True),     # the same with constants from LDS
+    (12288, 64, 1, 2, 12, 3070, True),    # three columns a phase
+    (704, 128, 1, 2, 34, 300, True),      # two waves a column
+    (6144, 128, 0, 2, 12, 6143, True),
+    (128, 104, 1, -1, 20, 1, True),
+    (3200, 72, 0, 3, 20, 1600, False),
+    (3264, 96, 1, 0, 20, 3200, True),
+    (32768, 64, 1, 2, 40, 21700, True),   # segments, the extraction column near a border
+    (32768, 64, 0, 3, 12, 32766, False),
+    (16384, 128, 1, 2, 33, 0, True),
+    (65536, 24, 0, 2, 12, 30000, False),
+    (11200, 96, 1, -2, 33, 5601, True),
 ]
 
 
@@ -101,12 +112,12 @@ def test_launch_shape_selects_the_stage_kernels():
         s.step(40)
         s.sync()
         assert np.array_equal(s.get_fields(), u)
-    p, u0, _ = setup(1024, 72, 1, 2, 4)
+    p, u0, _ = setup(1024, 136, 1, 2, 4)
     with start(p, u0, None, 4) as s:
-        assert not s.resident()  # a column does not fit a wave
+        assert not s.resident()  # a column does not fit two waves
 
 
-@pytest.mark.parametrize("N,M", [(1024, 32), (8192, 64)])
+@pytest.mark.parametrize("N,M", [(1024, 32), (8192, 64), (16384, 128)])
 def test_launch_that_gives_up_loses_no_step(N, M):
     """A wait of zero closes the launch's gate before any block can open it:
     the launch, and the ones queued behind it, change nothing, and the steps
@@ -159,10 +170,11 @@ def test_resident_solvers_on_several_threads():
         assert np.array_equal(got[i][0], ref[i]) and got[i][1], i
 
 
-BATCH = [  # N, M, m, steps, source: several row classes, narrow and wide tiles, one that does not fit
+BATCH = [  # N, M, m, steps, source: several row classes, narrow and wide tiles, two that do not fit
     (256, 16, 2, 40, True), (4096, 32, 2, 40, True), (8192, 32, -3, 33, False), (4096, 32, 0, 64, True),
     (16384, 32, 1, 20, False), (8192, 64, 2, 40, True), (2048, 64, 3, 12, False), (6080, 40, 2, 40, True),
-    (1024, 24, -1, 70, False), (512, 72, 2, 40, True),
+    (1024, 24, -1, 70, False), (512, 72, 2, 40, True), (2048, 128, 1, 33, True), (512, 136, 2, 40, True),
+    (32768, 48, 2, 20, True),
 ]
 
 
