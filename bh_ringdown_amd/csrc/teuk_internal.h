@@ -85,6 +85,7 @@ struct Ctl {
                        // bit 2: a resident launch stopped half way
   int fail;            // a resident launch gave up: later ones do nothing until
                        // the host has run the missing steps
+  unsigned ended;      // blocks of the current record launch that have ended
   double timer;        // solver time, advanced by repeated addition (body.cu:214)
   ResGate gate[2];
 };
