@@ -256,8 +256,8 @@ void host_source_prepare(const Grid &g, const SrcStep &st, SrcPrep &out) {
 // The fewest columns per block (a multiple of 8, so that the last block holds
 // at least 8 too: its edge columns and what the rho fill reads) that put the
 // grid on the chip with one block per CU: the narrowest tiles were the fastest
-// at every size (4096x32 RK4: 16 columns 2.9 us a stage, 32 3.0, 64 5.6;
-// 2048x64: 8 columns 3.6, 16 3.5, 32 6.2).  A tile that needs more than eight
+// at every size (4096x32 RK4: 16 columns 2.5 us a stage, 32 2.9, 64 5.1;
+// 2048x64: 8 columns 3.2, 16 3.5, 32 5.3).  A tile that needs more than eight
 // columns per thread, or more LDS than a CU has, does not fit; nor does a
 // column of more than 128 rows, which must lie within two waves.
 bool resident_shape(int N, int M, int cus, ResShape &sh) {
@@ -274,7 +274,7 @@ bool resident_shape(int N, int M, int cus, ResShape &sh) {
 
 // Measured time of one stage with tiles of kResCP[c] columns per thread (us).
 static double stage_us(int M, int c) {
-  static const double k32[5] = {2.8, 3.1, 5.4, 7.2, 8.8}, k64[5] = {3.3, 3.8, 6.0, 8.2, 10.4};
+  static const double k32[5] = {2.5, 2.9, 5.2, 7.2, 8.9}, k64[5] = {3.2, 3.5, 5.4, 7.6, 8.9};
   return M <= 32 ? k32[c] : k64[c];
 }
 
@@ -353,7 +353,7 @@ std::vector<ResGroup> resident_groups(const std::vector<std::pair<int, int>> &sh
       while (total(m, g.CP, want) > cus) want += 8;
       for (int i : m) g.C.push_back(tile(i, g.CP, want));
       g.members = std::move(m);
-      g.MT = g.CP >= 4 ? cls : 0;
+      g.MT = g.CP >= 4 || cls == 32 || cls == kWave ? cls : 0;   // (res_built_rows of all members)
       out.push_back(g);
     }
   }

@@ -199,7 +199,7 @@ TEUK_HD double *res_k8(const DevState &d, int N) { return d.scratch + 2 * (size_
 // 64, kAnyTall any of 65 to 128 (two waves a column).
 constexpr int kAnyTall = 1;
 TEUK_HD constexpr int res_built_rows(int M, int CP) {
-  if (CP < 4) return 0;
+  if (CP < 4) return M == 64 || M == 32 ? M : 0;
   return M == 128 || M == 64 || M == 32 ? M : (M > kWave ? kAnyTall : 0);
 }
 // Groups of M threads in a block: any threads for the small-tile kernel (at
@@ -207,12 +207,19 @@ TEUK_HD constexpr int res_built_rows(int M, int CP) {
 TEUK_HD constexpr int res_groups(int M, int CP) {
   return CP >= 4 ? (M > kWave ? 4 : (kResThreads / kWave) * (kWave / M)) : (M > kWave ? 0 : kResThreads / M);
 }
-// LDS of one block: columns of M + 1 rows of two complex fields (C + 8; C + 12
-// for the sweeping kernel of CP >= 4), the extraction integrals, the column
+// Whether tiles of one column per thread exchange edge columns after every
+// second stage only (0: no), and the columns per thread that the stage
+// between then takes.
+TEUK_HD constexpr int res_pair(int M, int C) {
+  const int G = kResThreads / M;
+  return C + 8 <= G ? 1 : (C <= G && G >= 16 ? 2 : 0);
+}
+// LDS of one block: columns of M + 1 rows of two complex fields (C + 16, twice;
+// C + 12 for the sweeping kernel of CP >= 4), the extraction integrals, the column
 // constants where they are not scalar loads.
 TEUK_HD constexpr bool res_uniform(int M, int CP) { return CP > 4 && M >= kWave; }
 TEUK_HD constexpr size_t res_lds_bytes(int M, int C, int CP) {
-  return (size_t)32 * (C + (CP >= 4 ? 12 : 8)) * (M + 1) + 32 * (size_t)M +
+  return (size_t)(CP >= 4 ? 32 * (C + 12) : 64 * (C + 16)) * (M + 1) + 32 * (size_t)M +
          (CP >= 4 && !res_uniform(M, CP) ? 64 * (size_t)C : 0);
 }
 // The narrowest tile: a sweep reads the halo on its far side in its second

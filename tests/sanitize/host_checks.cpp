@@ -168,7 +168,8 @@ void resident_tiles(int cus) {
       }
       const int rest = N - (sh.B - 1) * sh.C;
       const bool sweep = sh.CP >= 4;
-      const size_t xbytes = 2 * (size_t)sh.B * 8 * 32 * M, cbytes = sweep ? 24 * (size_t)N * M : 0;
+      const int edges = sh.CP == 1 && res_pair(M, sh.C) && sh.C >= 16 ? 16 : 8;   // columns a block publishes
+      const size_t xbytes = 2 * (size_t)sh.B * edges * 32 * M, cbytes = sweep ? 24 * (size_t)N * M : 0;
       const size_t NM32 = 32 * (size_t)N * M;
       const bool good = M >= 16 && M <= 128 && sh.B <= cus && sh.C % 8 == 0 && sh.C >= res_least_tile(M, sh.CP) && rest >= 8 && rest <= sh.C &&
                         res_groups(M, sh.CP) >= (sweep ? 4 : 8) && res_groups(M, sh.CP) * sh.CP >= sh.C &&

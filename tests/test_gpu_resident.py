@@ -208,3 +208,30 @@ def test_batch_of_resident_members_equal_alone(integrator, wait):
             assert np.array_equal(o["h"], out["h"]) and np.array_equal(o["t"], out["t"]), c
     for s in solvers:
         s.close()
+
+
+@pytest.mark.parametrize("c", [
+    (256, 16, 1, 2, 34, 0, True),         # exchange after every second stage; extraction in the rho edge fill
+    (6080, 16, 0, 3, 33, 6079, True),     # RK3 pairs across steps; the last block as narrow as the halo
+    (6080, 16, 1, 2, 20, 6077, False),
+    (704, 32, 0, 2, 35, 11, True),
+    (320, 24, 1, -1, 20, 318, True),      # rows that share a wave's lanes unevenly
+    (8192, 16, 0, 2, 20, 40, True),       # two columns for some threads in the stage between
+    (4096, 32, 1, -3, 33, 4095, True),
+    (4096, 24, 0, 2, 20, 17, False),
+    (1024, 48, 1, 2, 20, 9, True),        # every stage: one column per thread
+    (8192, 32, 0, 1, 20, 2, True),        # two
+    (1600, 56, 1, 2, 20, 1598, True),
+], ids=str)
+def test_small_tiles(c):
+    N, M, integrator, m, steps, je, source = c
+    p, u0, rows = setup(N, M, integrator, m, steps, je, source)
+    uo, psio, ho, dedto = oracle(p, u0, rows, steps)
+    with start(p, u0, rows, steps) as s:
+        for n in (1, steps - 4, 3):
+            s.step(n)
+        s.sync()
+        assert s.resident()
+        u, out, psi = s.get_fields(), s.output(), s.psi()
+    assert np.array_equal(u, uo) and np.array_equal(psi, psio)
+    assert np.array_equal(out["h"], ho) and np.array_equal(out["dedt"], dedto)
