@@ -292,12 +292,18 @@ hipError_t launch_resident_batch(const SolveDesc *descs, const ResBlock *blocks,
 
 // Launch shape for an N x M grid, from measurements on an MI355X: 2-row
 // wavefronts (2 + (M - 10) / 2 per strip, an odd count, so one wavefront per
-// block), compiled for 3 waves per SIMD from M = 64 up; 4-row wavefronts at
-// 8 M points and more, where there are wavefronts enough and fewer theta
+// block), compiled for 3 waves per SIMD from M = 64 up; 8-row ones on tall
+// grids past the last-level cache; 4-row wavefronts at 8 M points and more, where there are wavefronts enough and fewer theta
 // halo re-reads pay.
 Tiling default_tiling(int N, int M) {
   Tiling t;
   const bool large = (long long)N * M >= (1LL << 23);
+  // Between: the stages no longer live in the last-level cache, and on tall
+  // grids 8-row chunks, which re-read the fewest halo rows, win (2-row / 8-row,
+  // us a stage: 16000 x 256 SSP-RK3 91.2 / 85.0, RK4 99.6 / 94.7; 24576 x 192
+  // 105.2 / 100.0; 8192 x 512 93.2 / 88.7), not on lower ones (32768 x 136 95.0
+  // / 99.5) nor below (12288 x 256, 3.1 M points, 59.3 / 61.2).
+  if (!large && (long long)N * M >= 7 * (1LL << 19) && M >= 192) return Tiling{1, 2, 8};
   t.rows = large ? 4 : kDefaultThetaRows;
   t.wpe = (!large && M >= 64) ? 3 : 2;
   const int chunks = theta_chunks(M, t.rows);

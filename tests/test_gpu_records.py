@@ -50,3 +50,16 @@ def test_fields_round_trip(N, M, integrator):
         whole.set_fields(u0)
         whole.step(40)
         assert s.get_fields().tobytes() == whole.get_fields().tobytes()
+
+
+@pytest.mark.parametrize("N,M,integrator", [(14336, 256, 0), (19136, 192, 1), (7168, 512, 1)])
+def test_default_shape_of_tall_grids(N, M, integrator):
+    """The smallest grids whose default is 8-row chunks."""
+    p, u0, _ = setup(N, M, integrator, 2, 3, je=N // 2)
+    with teuk.Solver(p) as s:
+        s.set_fields(u0)
+        s.step(3)
+        s.sync()
+        u, psi = s.get_fields(), s.psi()
+    uo, psio, _, _ = oracle(p, u0, None, 3)
+    assert np.array_equal(u, uo) and np.array_equal(psi, psio)
