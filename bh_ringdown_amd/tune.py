@@ -23,6 +23,10 @@ tune_batch() times whole batch steps.  Winners are kept in a JSON cache
 (TEUK_TUNE_CACHE, default ~/.cache/bh_ringdown_amd/tuning.json) keyed by
 grid shape and integrator, and looked up by best_solver_tiling() /
 best_batch_tiling() / best_batch_groups().
+
+The shapes are those of the per-stage kernels, which step grids of more than
+128 theta rows.  Setting one on a smaller grid's solver or batch takes it off
+resident stepping, which is the faster there.
 """
 import itertools
 import json
