@@ -21,9 +21,6 @@ using namespace teuk;
 
 struct teuk_batch;
 
-// Longest a resident launch waits for all of its blocks to be on the GPU (s).
-constexpr double kResidentWait = 0.25;
-
 struct teuk_solver {
   teuk_params P;
   Grid g;
@@ -33,7 +30,7 @@ struct teuk_solver {
   // the chip, a launch shape was set for the stage kernels, or a launch gave up.
   bool resident = false;
   ResShape res_shape{0, 0, 0};
-  double res_wait = kResidentWait;
+  double res_wait = kResWait;
   int gate = 0;                  // which of the control block's two gates is next
   bool res_pending = false;      // resident launches since the control block was last read
   // Grids beyond the chip: stepped in segments (resident_segments), from the
@@ -192,8 +189,6 @@ void chain_forget(hipStream_t stream) {
   }
 }
 
-long long wait_ticks(double seconds) { return seconds > 0.0 ? (long long)(seconds * 1e8) + 1 : 0; }
-
 // CUs of the current device (asked of the runtime once per device).
 int device_cus() {
   static std::mutex lock;
@@ -304,7 +299,7 @@ int resident_steps(teuk_solver *s, int n) {
     auto launch = [&](const ResShape &sh, const ResSpan &sp, ResGate *gate) {
       return resident_launch(s->stream, [&]() {
         return launch_resident(s->g, s->d, s->P.integrator, s->has_src, sh, sp, m, s->nt, gate,
-                               wait_ticks(s->res_wait), s->stream);
+                               res_wait_ticks(s->res_wait), s->stream);
       });
     };
     int rc = TEUK_OK;
@@ -1273,7 +1268,7 @@ int batch_rebuild(teuk_batch *b) {
     g.CP = rg.CP;
     g.MT = rg.MT;
     g.block_off = blocks.size();
-    g.wait = kResidentWait;
+    g.wait = kResWait;
     for (size_t m = 0; m < rg.members.size(); m++) {
       teuk_solver *s = fit[rg.members[m]];
       const int C = rg.C[m];
@@ -1411,7 +1406,7 @@ int batch_resident(teuk_batch *b, const teuk_batch::Group &g, int nsteps) {
     ResGate *gate = b->gates + b->gate, *other = b->gates + (b->gate ^ 1);
     const int rc = resident_launch(b->stream, [&]() {
       return launch_resident_batch(descs, b->d_blocks + g.block_off, g.nblocks, b->integrator, g.CP, g.MT, g.lds, m,
-                                   gate, wait_ticks(g.wait), b->stream);
+                                   gate, res_wait_ticks(g.wait), b->stream);
     });
     if (rc) return rc;
     HIPCHK(launch_finalize_batch(descs, g.count, m, gate, other, b->stream));
@@ -1765,7 +1760,7 @@ int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *th
       const int n = std::min(kRing, nsteps - done);
       if (has_src) HIPCHK(launch_source(g, d, 0, n, true, st));
       HIPCHK(launch_resident(g, d, p->integrator, has_src, sh, ResSpan{0, p->N, 0, p->N, d.U, d.D, nullptr, 0}, n, nsteps,
-                             d.ctl->gate + gate, wait_ticks(kResidentWait), st));
+                             d.ctl->gate + gate, res_wait_ticks(kResWait), st));
       HIPCHK(launch_finalize(g, d, n, d.ctl->gate + gate, d.ctl->gate + (gate ^ 1), st));
     }
     HIPCHK(hipStreamSynchronize(st));

@@ -227,6 +227,15 @@ TEUK_HD constexpr size_t res_lds_bytes(int M, int C, int CP) {
 TEUK_HD constexpr int res_least_tile(int M, int CP) { return CP >= 4 ? ((res_groups(M, CP) * (CP / 2) + 11) & ~7) : 8; }
 constexpr size_t kResLdsMax = 163840 - 512;   // a CU's LDS less the kernel's static part
 constexpr int kResCP[5] = {1, 2, 4, 6, 8};
+// A launch's longest wait for all of its blocks to be on the GPU (s), unless
+// one is given, and the longest it takes: a launch must end in bounded time,
+// also where two processes each hold CUs that the other waits for.
+constexpr double kResWait = 0.25, kResWaitMost = 60.0;
+// That wait in the GPU's 100 MHz ticks; 0: it does not wait.
+inline long long res_wait_ticks(double seconds) {
+  if (!(seconds > 0.0)) return 0;
+  return (long long)((seconds < kResWaitMost ? seconds : kResWaitMost) * 1e8) + 1;
+}
 // The launch shape for an N x M grid on `cus` CUs, or false if its fields do
 // not fit on the chip.
 bool resident_shape(int N, int M, int cus, ResShape &sh);

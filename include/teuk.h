@@ -200,8 +200,9 @@ int teuk_set_theta_rows(teuk_solver *s, int rows);
  * million points whole, larger ones in segments of rho columns, one after
  * the other, where that is faster.  Such a launch needs all of its blocks on
  * the GPU at once.  If it does not get them within `seconds` (0.25 by default; 0: it
- * never waits), because another process holds the CUs, it changes nothing,
- * and its steps and all later ones are run by the stage kernels.  Results do
+ * never waits; at most 60, which larger values are taken as), because another
+ * process holds the CUs, it changes nothing, and its steps and all later ones
+ * are run by the stage kernels.  Results do
  * not depend on it. */
 int teuk_set_resident_wait(teuk_solver *s, double seconds);
 /* *on: 1 while the solver's next steps would be resident ones, else 0. */

@@ -255,9 +255,26 @@ void resident_batches(int cus) {
   }
 }
 
+// A resident launch's wait in ticks: none for 0, else positive and bounded
+// for every number of seconds.
+void resident_waits() {
+  using namespace teuk;
+  const long long most = (long long)(kResWaitMost * 1e8) + 1;
+  bool good = res_wait_ticks(0.0) == 0 && res_wait_ticks(0.25) == 25000001 && res_wait_ticks(5e-324) == 1;
+  for (double s : {1e-9, 59.9, 60.0, 61.0, 9.3e10, 1e300, (double)INFINITY}) {
+    const long long t = res_wait_ticks(s);
+    good = good && t >= 1 && t <= most && (s < kResWaitMost || t == most);
+  }
+  if (!good) {
+    std::printf("bad resident wait\n");
+    failures++;
+  }
+}
+
 }  // namespace
 
 int main() {
+  resident_waits();
   chunk_layout_and_block_order();
   grids_and_tables(1024, 32, -100.0, 300.0, 0.5, 2.0);
   grids_and_tables(512, 16, -40.0, 60.0, 0.99, -3.0);

@@ -1,0 +1,31 @@
+"""The wait of resident launches for their blocks (teuk_set_resident_wait):
+what a solver, a batch and the no-allocation call do with values from zero to
+infinity, set before the first step or between steps."""
+import math
+
+import numpy as np
+import pytest
+
+from bh_ringdown_amd import teuk
+from tests.test_gpu_resident import setup, start
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("seconds", [5e-3, 3600.0, 1e11, 1e300, math.inf])
+def test_a_long_wait_is_not_taken_as_none(seconds):
+    p, u0, _ = setup(1024, 32, 1, 2, 40)
+    with start(p, u0, None, 40) as s:
+        s.set_resident_wait(seconds)
+        s.step(40)
+        s.sync()
+        assert s.resident()
+
+
+@pytest.mark.parametrize("seconds", [-1.0, -math.inf, math.nan])
+def test_what_is_no_wait_is_refused(seconds):
+    p, u0, _ = setup(128, 16, 1, 2, 4)
+    with start(p, u0, None, 4) as s:
+        with pytest.raises(teuk.TeukError) as e:
+            s.set_resident_wait(seconds)
+        assert e.value.code == teuk.TEUK_EINVAL
