@@ -1185,6 +1185,7 @@ int teuk_set_tiling(teuk_solver *s, int waves_per_block, int waves_per_eu) {
 int teuk_set_resident_wait(teuk_solver *s, double seconds) {
   if (!s || !(seconds >= 0.0)) return TEUK_EINVAL;
   s->res_wait = seconds;
+  if (s->batch) s->batch->dirty = true;   // its group waits as long as its least patient member
   return TEUK_OK;
 }
 
@@ -1268,18 +1269,19 @@ int batch_rebuild(teuk_batch *b) {
     g.CP = rg.CP;
     g.MT = rg.MT;
     g.block_off = blocks.size();
-    g.wait = kResWait;
+    std::vector<double> waits;
     for (size_t m = 0; m < rg.members.size(); m++) {
       teuk_solver *s = fit[rg.members[m]];
       const int C = rg.C[m];
       if (s->has_src) g.max_cells = std::max(g.max_cells, s->P.ptsx * s->P.ptsy);
       g.lds = std::max(g.lds, res_lds_bytes(s->P.M, C, rg.CP));
-      g.wait = std::min(g.wait, s->res_wait);
+      waits.push_back(s->res_wait);
       const int B = (s->P.N + C - 1) / C;
       for (int k = 0; k < B; k++) blocks.push_back(ResBlock{(int)hd.size() - g.first, k, C, B});
       hd.push_back(describe(s));
     }
     g.nblocks = (int)(blocks.size() - g.block_off);
+    g.wait = res_shared_wait(waits);
     b->groups.push_back(g);
   }
   const size_t first_stage = b->groups.size();

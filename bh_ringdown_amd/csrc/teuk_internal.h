@@ -236,6 +236,12 @@ inline long long res_wait_ticks(double seconds) {
   if (!(seconds > 0.0)) return 0;
   return (long long)((seconds < kResWaitMost ? seconds : kResWaitMost) * 1e8) + 1;
 }
+// The wait of a launch that members with these waits share.
+inline double res_shared_wait(const std::vector<double> &waits) {
+  double w = kResWaitMost;
+  for (double x : waits) w = x < w ? x : w;
+  return w;
+}
 // The launch shape for an N x M grid on `cus` CUs, or false if its fields do
 // not fit on the chip.
 bool resident_shape(int N, int M, int cus, ResShape &sh);

@@ -202,8 +202,8 @@ int teuk_set_theta_rows(teuk_solver *s, int rows);
  * the GPU at once.  If it does not get them within `seconds` (0.25 by default; 0: it
  * never waits; at most 60, which larger values are taken as), because another
  * process holds the CUs, it changes nothing, and its steps and all later ones
- * are run by the stage kernels.  Results do
- * not depend on it. */
+ * are run by the stage kernels.  A launch that members of a batch share
+ * waits as long as the shortest of their waits.  Results do not depend on it. */
 int teuk_set_resident_wait(teuk_solver *s, double seconds);
 /* *on: 1 while the solver's next steps would be resident ones, else 0. */
 int teuk_resident(teuk_solver *s, int *on);

@@ -265,6 +265,8 @@ void resident_waits() {
     const long long t = res_wait_ticks(s);
     good = good && t >= 1 && t <= most && (s < kResWaitMost || t == most);
   }
+  good = good && res_shared_wait({10.0, 2.0, 30.0}) == 2.0 && res_shared_wait({5.0}) == 5.0 &&
+         res_shared_wait({kResWait, 0.0}) == 0.0;
   if (!good) {
     std::printf("bad resident wait\n");
     failures++;

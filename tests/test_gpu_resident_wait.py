@@ -29,3 +29,38 @@ def test_what_is_no_wait_is_refused(seconds):
         with pytest.raises(teuk.TeukError) as e:
             s.set_resident_wait(seconds)
         assert e.value.code == teuk.TEUK_EINVAL
+
+
+def batch_of(specs, steps):
+    solvers = [start(p, u0, None, steps) for p, u0, _ in specs]
+    b = teuk.Batch(integrator=1)
+    for s in solvers:
+        assert b.add(s)
+    return b, solvers
+
+
+def test_wait_set_between_the_steps_of_a_batch():
+    """It holds from the next step on: a wait of zero makes that launch give
+    up, and no step is lost."""
+    specs = [setup(1024, 32, 1, m, 96, seed=m) for m in (1, 2)]
+    ref = []
+    for p, u0, _ in specs:
+        with start(p, u0, None, 96) as s:
+            s.step(96)
+            s.sync()
+            ref.append(s.get_fields())
+    b, solvers = batch_of(specs, 96)
+    b.step(32)
+    b.sync()
+    assert all(s.resident() for s in solvers)
+    solvers[1].set_resident_wait(0.0)
+    b.step(32)
+    b.sync()
+    assert not any(s.resident() for s in solvers)      # they shared the launch
+    b.step(32)
+    b.sync()
+    for s, u in zip(solvers, ref):
+        assert s.progress()[0] == 96 and np.array_equal(s.get_fields(), u)
+    b.close()
+    for s in solvers:
+        s.close()
