@@ -108,6 +108,11 @@ struct teuk_batch {
 
 namespace {
 
+// Whether a batch steps a member by resident launches: those it fits in whole.
+bool batch_resident_member(const teuk_batch *b, const teuk_solver *s) {
+  return b->resident && s->resident && s->segs.spans.empty();
+}
+
 // The stream that runs a solver's steps: its own, or its batch's.
 hipStream_t run_stream(const teuk_solver *s) { return s->batch ? s->batch->stream : s->stream; }
 
@@ -1192,7 +1197,7 @@ int teuk_set_resident_wait(teuk_solver *s, double seconds) {
 int teuk_resident(teuk_solver *s, int *on) {
   if (!s || !on) return TEUK_EINVAL;
   if (const int rc = settle(s)) return rc;
-  *on = s->resident ? 1 : 0;
+  *on = (s->batch ? batch_resident_member(s->batch, s) : s->resident) ? 1 : 0;
   return TEUK_OK;
 }
 
@@ -1259,7 +1264,7 @@ int batch_rebuild(teuk_batch *b) {
   std::vector<teuk_solver *> fit, rest;
   for (teuk_solver *s : b->members)
     if (s->k_host < member_steps(s))
-      (b->resident && s->resident && s->segs.spans.empty() ? fit : rest).push_back(s);
+      (batch_resident_member(b, s) ? fit : rest).push_back(s);
   std::vector<std::pair<int, int>> shapes;
   for (teuk_solver *s : fit) shapes.push_back({s->P.N, s->P.M});
   for (const ResGroup &rg : resident_groups(shapes, device_cus())) {

@@ -205,7 +205,8 @@ int teuk_set_theta_rows(teuk_solver *s, int rows);
  * are run by the stage kernels.  A launch that members of a batch share
  * waits as long as the shortest of their waits.  Results do not depend on it. */
 int teuk_set_resident_wait(teuk_solver *s, double seconds);
-/* *on: 1 while the solver's next steps would be resident ones, else 0. */
+/* *on: 1 while the solver's next steps would be resident ones, else 0; for a
+ * solver in a batch, the batch's next steps of it. */
 int teuk_resident(teuk_solver *s, int *on);
 
 /* The 12 per-step source coefficients (the canonical T_4 coefficients times

@@ -1,6 +1,7 @@
 """The wait of resident launches for their blocks (teuk_set_resident_wait):
 what a solver, a batch and the no-allocation call do with values from zero to
-infinity, set before the first step or between steps."""
+infinity, set before the first step or between steps; and what
+teuk_resident says of a batch's members."""
 import math
 
 import numpy as np
@@ -62,5 +63,22 @@ def test_wait_set_between_the_steps_of_a_batch():
     for s, u in zip(solvers, ref):
         assert s.progress()[0] == 96 and np.array_equal(s.get_fields(), u)
     b.close()
+    for s in solvers:
+        s.close()
+
+
+def test_resident_of_members():
+    """A member that is stepped in segments alone goes by stages in a batch;
+    with a launch shape set for the batch all of them do."""
+    specs = [setup(1024, 32, 1, 2, 8), setup(32768, 64, 1, 2, 8), setup(512, 136, 1, 2, 8)]
+    b, solvers = batch_of(specs, 8)
+    assert [s.resident() for s in solvers] == [True, False, False]
+    b.step(4)
+    b.sync()
+    assert [s.resident() for s in solvers] == [True, False, False]
+    b.set_tiling(1, 2, 0, 32, theta_rows=2)
+    assert not any(s.resident() for s in solvers)
+    b.close()
+    assert [s.resident() for s in solvers] == [True, True, False]      # alone again
     for s in solvers:
         s.close()
