@@ -108,6 +108,12 @@ struct teuk_batch {
 
 namespace {
 
+// What a control block says of its solve.
+int solve_code(const Ctl &c) {
+  if (c.status & 4) return TEUK_ESTALLED;
+  return c.status ? TEUK_EDIVERGED : TEUK_OK;
+}
+
 // Whether a batch steps a member by resident launches: those it fits in whole.
 bool batch_resident_member(const teuk_batch *b, const teuk_solver *s) {
   return b->resident && s->resident && s->segs.spans.empty();
@@ -523,6 +529,7 @@ const char *teuk_strerror(int code) {
     case TEUK_EINVAL: return "invalid argument or unsupported size";
     case TEUK_EHIP: return "HIP runtime error";
     case TEUK_ENOMEM: return "out of memory";
+    case TEUK_ESTALLED: return "blocks of a launch stopped waiting for each other (the solve's fields are lost)";
     case TEUK_EDIVERGED: return "non-finite field (solve diverged)";
     case TEUK_EIO: return "trajectory or waveform file error";
     case TEUK_ERANGE: return "step beyond the scheduled run or trajectory";
@@ -696,6 +703,7 @@ void fill_init(const teuk_params *p, const double *r_c, const double *theta, con
   c0.nrec = 0;
   c0.status = 0;
   c0.timer = 0.0;
+  c0.reads = kResReads;
   std::memcpy(stage + L.ctl, &c0, sizeof(Ctl));
   if (stag) {  // Old/kern.cu:90-135: the same fields at rho - dx/2 with r_h
     host_source_phase(N, p->mass, p->a, p->m, r_h, at(L.phase_h));
@@ -996,7 +1004,7 @@ int teuk_sync(teuk_solver *s) {
   const int rc = read_ctl(s, c);
   if (rc) return rc;
   if (s->timing) flush_timing(s);
-  return c.status ? TEUK_EDIVERGED : TEUK_OK;
+  return solve_code(c);
 }
 
 int teuk_status(teuk_solver *s) {
@@ -1004,7 +1012,7 @@ int teuk_status(teuk_solver *s) {
   Ctl c;
   const int rc = read_ctl(s, c);
   if (rc) return rc;
-  return c.status ? TEUK_EDIVERGED : TEUK_OK;
+  return solve_code(c);
 }
 
 int teuk_progress(teuk_solver *s, int *k, double *t) {
@@ -1191,6 +1199,14 @@ int teuk_set_resident_wait(teuk_solver *s, double seconds) {
   if (!s || !(seconds >= 0.0)) return TEUK_EINVAL;
   s->res_wait = seconds;
   if (s->batch) s->batch->dirty = true;   // its group waits as long as its least patient member
+  return TEUK_OK;
+}
+
+int teuk_set_exchange_reads(teuk_solver *s, int reads) {
+  if (!s || reads < 0) return TEUK_EINVAL;
+  if (const int rc = settle(s)) return rc;
+  HIPCHK(hipStreamSynchronize(run_stream(s)));
+  HIPCHK(hipMemcpy(&s->d.ctl->reads, &reads, sizeof reads, hipMemcpyHostToDevice));
   return TEUK_OK;
 }
 
@@ -1581,7 +1597,8 @@ int teuk_batch_sync(teuk_batch *b) {
     Ctl c;
     const int r = read_ctl(s, c);
     if (r) return r;
-    if (c.status) rc = TEUK_EDIVERGED;
+    const int code = solve_code(c);
+    if (code == TEUK_ESTALLED || rc == TEUK_OK) rc = code;
   }
   return rc;
 }
@@ -1800,5 +1817,5 @@ int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *th
     }
   }
   if (nrows) *nrows = cnt;
-  return c.status ? TEUK_EDIVERGED : TEUK_OK;
+  return solve_code(c);
 }

@@ -76,16 +76,20 @@ struct ResGate {
   int decision;
 };
 
+// The most reads of a neighbour's flag in one wait, about a microsecond each.
+constexpr int kResReads = 1 << 22;
+
 // Device control block, one per solver.
 struct Ctl {
   int k;               // completed steps
   int nrec;            // output records written
   int status;          // 0 ok; bit 0: non-finite Psi at the extraction column,
                        // bit 1: the whole-field sentinel fired (see kGrowthLimit),
-                       // bit 2: a resident launch stopped half way
+                       // bit 2: a resident launch stopped half way (its fields are no state)
   int fail;            // a resident launch gave up: later ones do nothing until
                        // the host has run the missing steps
   unsigned ended;      // blocks of the current record launch that have ended
+  int reads;           // a resident launch's reads of a neighbour's flag in one wait (kResReads)
   double timer;        // solver time, advanced by repeated addition (body.cu:214)
   ResGate gate[2];
 };

@@ -53,13 +53,15 @@ class Result:
     points: int = 0
     records: dict = field(default_factory=dict)     # output(): k, t, dedt, h
     psi: np.ndarray = None
-    failed: bool = False    # retired by the divergence sentinel (records up to the failure)
+    failed: bool = False    # retired by the divergence sentinel or stalled (records up to the failure)
 
     @property
     def latency(self):
         return self.done - self.arrival
 
 
+# one solve's failure, not the GPU's or the caller's
+SOLVE_FAILED = (teuk.TEUK_EDIVERGED, teuk.TEUK_ESTALLED)
 MAX_IOTA = math.radians(85.0)   # the trajectory generator's limit (polar passes excluded)
 
 
@@ -262,14 +264,14 @@ class Server:
                     batch.sync()
                     any_failed = False
                 except teuk.TeukError as e:
-                    if e.code != teuk.TEUK_EDIVERGED:
+                    if e.code not in SOLVE_FAILED:
                         raise
                     any_failed = True
                 st["sync_s"] += clock() - ts
                 ts = clock()
                 for rid in list(live):
                     req, p, s, nread, outs, psis = live[rid]
-                    if any_failed and s.status() == teuk.TEUK_EDIVERGED:
+                    if any_failed and s.status() in SOLVE_FAILED:
                         res = results[rid]
                         res.failed = True
                         res.done = now()
@@ -366,7 +368,7 @@ def run_plain(requests, clock=time.perf_counter, integrator=1, deadline=None, st
                 try:
                     s.sync()
                 except teuk.TeukError as e:
-                    if e.code != teuk.TEUK_EDIVERGED:
+                    if e.code not in SOLVE_FAILED:
                         raise
                     res.failed = True
                 done_steps += k

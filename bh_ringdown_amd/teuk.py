@@ -20,7 +20,7 @@ PI15 = 3.14159265358979  # parm.h:12
 _dp = ctypes.POINTER(ctypes.c_double)
 
 TEUK_OK, TEUK_EINVAL, TEUK_EHIP, TEUK_ENOMEM, TEUK_EDIVERGED, TEUK_EIO, TEUK_ERANGE = 0, -1, -2, -3, -4, -5, -6
-TEUK_ETOOBIG = -7
+TEUK_ETOOBIG, TEUK_ESTALLED = -7, -8
 NOALLOC_BYTES = 64 << 20
 
 
@@ -77,7 +77,7 @@ EXPORTS = [
     "teuk_batch_remove", "teuk_batch_set_tiling", "teuk_batch_step", "teuk_batch_sync", "teuk_batch_info",
     "teuk_source_coeffs", "teuk_source_patch", "teuk_grid_half", "teuk_create_staggered",
     "teuk_trajectory_schedule_staggered", "teuk_status", "teuk_solve_noalloc", "teuk_batch_set_cache_groups",
-    "teuk_ot_transition", "teuk_set_resident_wait", "teuk_resident", "teuk_set_theta_rows", "teuk_batch_set_theta_rows",
+    "teuk_ot_transition", "teuk_set_resident_wait", "teuk_set_exchange_reads", "teuk_resident", "teuk_set_theta_rows", "teuk_batch_set_theta_rows",
 ]
 
 _lib = None
@@ -133,6 +133,7 @@ def lib():
         "teuk_set_theta_rows": ([vp, ctypes.c_int], ctypes.c_int),
         "teuk_resident": ([vp, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
         "teuk_set_resident_wait": ([vp, ctypes.c_double], ctypes.c_int),
+        "teuk_set_exchange_reads": ([vp, ctypes.c_int], ctypes.c_int),
         "teuk_batch_set_theta_rows": ([vp, ctypes.c_int], ctypes.c_int),
         "teuk_ot_transition": ([ctypes.c_double, _dp, _dp], ctypes.c_int),
         "teuk_remaining": ([vp, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
@@ -312,9 +313,9 @@ class Solver:
         _check(lib().teuk_sync(self._h), "teuk_sync")
 
     def status(self):
-        """TEUK_OK, or TEUK_EDIVERGED once the solve has failed (teuk_status)."""
+        """TEUK_OK, or TEUK_EDIVERGED or TEUK_ESTALLED once the solve has failed (teuk_status)."""
         rc = lib().teuk_status(self._h)
-        if rc not in (TEUK_OK, TEUK_EDIVERGED):
+        if rc not in (TEUK_OK, TEUK_EDIVERGED, TEUK_ESTALLED):
             _check(rc, "teuk_status")
         return rc
 
@@ -354,6 +355,10 @@ class Solver:
     def set_resident_wait(self, seconds):
         """Longest wait of a resident launch for its blocks (teuk_set_resident_wait)."""
         _check(lib().teuk_set_resident_wait(self._h, float(seconds)), "teuk_set_resident_wait")
+
+    def set_exchange_reads(self, reads):
+        """Reads of a neighbour's flag in one wait of a resident launch (teuk_set_exchange_reads)."""
+        _check(lib().teuk_set_exchange_reads(self._h, int(reads)), "teuk_set_exchange_reads")
 
     def resident(self):
         """Whether the next steps keep the fields on the chip (teuk_resident)."""
@@ -456,8 +461,8 @@ class Batch:
 def solve_noalloc(p, r_c, theta, nsteps, u0=None, steps=None, max_rows=None):
     """teuk_solve_noalloc: a whole solve in the library's fixed scratch memory.
     Returns (code, fields[4, M, N], records as Solver.output()); code is
-    TEUK_OK, TEUK_EDIVERGED or TEUK_ETOOBIG (then fields and records are
-    empty); other errors raise."""
+    TEUK_OK, TEUK_EDIVERGED, TEUK_ESTALLED or TEUK_ETOOBIG (then fields and
+    records are empty); other errors raise."""
     r_c = np.ascontiguousarray(r_c, dtype=np.float64)
     theta = np.ascontiguousarray(theta, dtype=np.float64)
     if u0 is not None and np.shape(u0) != (4, p.M, p.N):
@@ -475,7 +480,7 @@ def solve_noalloc(p, r_c, theta, nsteps, u0=None, steps=None, max_rows=None):
     n = ctypes.c_int()
     rc = lib().teuk_solve_noalloc(ctypes.byref(p), _ptr(r_c), _ptr(theta), u0p, arr, int(nsteps), _ptr(u), rows,
                                   cap, ctypes.byref(n))
-    if rc not in (TEUK_OK, TEUK_EDIVERGED, TEUK_ETOOBIG):
+    if rc not in (TEUK_OK, TEUK_EDIVERGED, TEUK_ESTALLED, TEUK_ETOOBIG):
         _check(rc, "teuk_solve_noalloc")
     k = n.value
     out = {"k": np.array([rows[i].k for i in range(k)], dtype=np.int64),

@@ -32,6 +32,10 @@ extern "C" {
 #define TEUK_ETOOBIG    -7   /* more memory than teuk_solve_noalloc's fixed
                                 scratch (TEUK_NOALLOC_BYTES)                 */
 
+#define TEUK_ESTALLED   -8   /* the solve is lost: a block of a launch stopped
+                                while its neighbours waited for it (see
+                                teuk_set_exchange_reads)                     */
+
 /* ---- run parameters ---------------------------------------------------- */
 /* Field names follow parm.h:1-11 and main.c:55-61 of the reference. */
 typedef struct teuk_params {
@@ -140,11 +144,12 @@ int teuk_trajectory_schedule_staggered(const double *rows, int nrows, int nsteps
  * followed by its edge fill).  Asynchronous on the solver's stream; use
  * teuk_sync. */
 int teuk_step(teuk_solver *s, int nsteps);
-/* Waits for the solver's queued steps; TEUK_EDIVERGED once the solve has
- * failed (see teuk_status). */
+/* Waits for the solver's queued steps; TEUK_EDIVERGED or TEUK_ESTALLED once the
+ * solve has failed (see teuk_status). */
 int teuk_sync(teuk_solver *s);
 
-/* TEUK_OK, or TEUK_EDIVERGED once this solve has failed: after each chunk
+/* TEUK_OK, or once this solve has failed TEUK_EDIVERGED (or TEUK_ESTALLED, see
+ * teuk_set_exchange_reads): after each chunk
  * of steps (at most 32, or one teuk_step call) a device sentinel checks
  * every value of the fields for non-finite values and magnitudes above
  * 1e60, and each step checks Psi at the extraction column.  Works alone or
@@ -205,6 +210,12 @@ int teuk_set_theta_rows(teuk_solver *s, int rows);
  * are run by the stage kernels.  A launch that members of a batch share
  * waits as long as the shortest of their waits.  Results do not depend on it. */
 int teuk_set_resident_wait(teuk_solver *s, double seconds);
+/* Blocks of a resident launch wait for each other's edge columns.  A wait ends
+ * after about `reads` reads of the neighbour's flag (2^22 by default, some
+ * seconds of them), which it reaches only if a block has stopped; the solve
+ * then fails with TEUK_ESTALLED.  Time in which the launch is not on the GPU
+ * does not count. */
+int teuk_set_exchange_reads(teuk_solver *s, int reads);
 /* *on: 1 while the solver's next steps would be resident ones, else 0; for a
  * solver in a batch, the batch's next steps of it. */
 int teuk_resident(teuk_solver *s, int *on);
@@ -263,8 +274,8 @@ int teuk_batch_set_theta_rows(teuk_batch *b, int rows);
 int teuk_batch_set_cache_groups(teuk_batch *b, long long group_bytes);
 /* Advance every unfinished member by up to nsteps steps (asynchronous). */
 int teuk_batch_step(teuk_batch *b, int nsteps);
-/* Waits for the batch; TEUK_EDIVERGED if any member has failed (find which
- * with teuk_status on each). */
+/* Waits for the batch; TEUK_EDIVERGED or TEUK_ESTALLED if any member has failed
+ * (find which with teuk_status on each). */
 int teuk_batch_sync(teuk_batch *b);
 int teuk_batch_info(teuk_batch *b, int *members, int *active, long long *bytes_used);
 
@@ -315,7 +326,7 @@ int teuk_traj_plunge(double a, double eta, double iota, double r0_over_isco, dou
  * Calls are serialised by a process-wide lock (they share the scratch, which
  * keeps the last call's contents; each call clears what must start at
  * zero).  Runs on the current device's null stream and returns when done;
- * TEUK_EDIVERGED if the sentinel fired. */
+ * TEUK_EDIVERGED if the sentinel fired, TEUK_ESTALLED as for teuk_sync. */
 #define TEUK_NOALLOC_BYTES (64LL << 20)
 int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *theta,
                        const double *u0, const teuk_source_step *steps, int nsteps,

@@ -243,3 +243,33 @@ def test_batch_schedule_lookup(tmp_path, monkeypatch):
     assert tune.best_batch_tiling([(4096, 32)] * 8)["chunk"] == e["chunk"]   # same shapes, other count
     assert tune.best_batch_groups([(4096, 32)] * 8) == 0                     # groups only for the tuned batch
     assert tune.best_batch_tiling([(2048, 16)]) is None
+
+
+def test_server_retires_a_stalled_solve_too(monkeypatch):
+    """A solve lost because its launch's blocks stopped is retired on its own,
+    as a diverged one is; an error of the batch itself still ends the run."""
+    from bh_ringdown_amd import teuk
+    reqs = [serve.Request(id=i, arrival=0.0, a=0.5, m=2, iota=0.1, eta=1e-3, N=4096, M=32, t_final=20.0, seed=i)
+            for i in range(3)]
+
+    class Stalling(_FakeSolver):
+        def status(self):
+            return teuk.TEUK_ESTALLED if self.fail_at is not None and self.k >= self.fail_at else teuk.TEUK_OK
+
+    class Batch(_FakeBatch):
+        code = teuk.TEUK_ESTALLED
+
+        def sync(self):
+            if any(s.status() != teuk.TEUK_OK for s in self.members):
+                raise teuk.TeukError(self.code, "teuk_batch_sync")
+
+    monkeypatch.setattr(serve, "prepare_host", _fake_host)
+    monkeypatch.setattr(serve, "prepare_device",
+                        lambda p, req, th, rows: (p, Stalling(p, fail_at=30 if req.id == 1 else None)))
+    monkeypatch.setattr(serve.teuk, "Batch", Batch)
+    srv = serve.Server(hbm_budget=1 << 40, chunk=16, target_points=1 << 30)
+    res = srv.run(reqs)
+    assert [res[i].failed for i in range(3)] == [False, True, False] and srv.stats["failed"] == 1
+    Batch.code = teuk.TEUK_EHIP
+    with pytest.raises(teuk.TeukError):
+        serve.Server(hbm_budget=1 << 40, chunk=16, target_points=1 << 30).run(reqs)
