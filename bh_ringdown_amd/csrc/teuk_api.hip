@@ -162,10 +162,16 @@ int scheduled_steps(const teuk_params *p) { return (int)(p->T / p->dt); }
 // launch on another stream than the last one's first waits for the event
 // recorded behind that.  One chain per device.  (Other processes' launches
 // can still hold CUs; the launch's own gate bounds that wait.)
+//
+// teuk_solve_noalloc must not create the event: until another solve has, its
+// launches (on the null stream) are not recorded, and the event is then first
+// recorded behind them.
 struct ResidentChain {
   std::mutex lock;
   hipEvent_t done = nullptr;
+  bool recorded = false;         // `done` is behind the last launch, which was on stream `last`
   hipStream_t last = nullptr;
+  bool unrecorded = false;       // launches on the null stream before there was an event
 };
 constexpr int kMaxDevices = 64;
 ResidentChain g_chain[kMaxDevices];
@@ -178,25 +184,38 @@ ResidentChain *resident_chain() {
 }
 
 template <class Launch>
-int resident_launch(hipStream_t stream, Launch launch) {
+int resident_launch(hipStream_t stream, Launch launch, bool may_create = true) {
   ResidentChain *chain = resident_chain();
   if (!chain) return TEUK_EHIP;
   ResidentChain &c = *chain;
   std::lock_guard<std::mutex> hold(c.lock);
-  if (!c.done) HIPCHK(hipEventCreateWithFlags(&c.done, hipEventDisableTiming));
-  if (c.last && c.last != stream) HIPCHK(hipStreamWaitEvent(stream, c.done, 0));
+  if (!c.done && may_create) {
+    HIPCHK(hipEventCreateWithFlags(&c.done, hipEventDisableTiming));
+    if (c.unrecorded) {
+      HIPCHK(hipEventRecord(c.done, nullptr));
+      c.recorded = true;
+      c.last = nullptr;
+      c.unrecorded = false;
+    }
+  }
+  if (c.recorded && c.last != stream) HIPCHK(hipStreamWaitEvent(stream, c.done, 0));
   HIPCHK(launch());
+  if (!c.done) {
+    c.unrecorded = true;
+    return TEUK_OK;
+  }
   HIPCHK(hipEventRecord(c.done, stream));
+  c.recorded = true;
   c.last = stream;
   return TEUK_OK;
 }
 
-// A stream about to be destroyed (idle): the chain's event has completed, and
-// a new stream may get its handle.
+// A stream about to be destroyed (idle): the chain's event has completed if
+// it is the last one's, and a new stream may get its handle.
 void chain_forget(hipStream_t stream) {
   for (ResidentChain &c : g_chain) {
     std::lock_guard<std::mutex> hold(c.lock);
-    if (c.last == stream) c.last = nullptr;
+    if (c.recorded && c.last == stream) c.recorded = false;
   }
 }
 
@@ -1772,23 +1791,26 @@ int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *th
   ResShape sh{0, 0, 0};
   Ctl c;
   if (nsteps < (1 << 28) && resident_shape(p->N, p->M, device_cus(), sh)) {
-    // This solve's place in the chain of resident launches is held until its
-    // last one has ended: that takes no event.
-    ResidentChain *chain = resident_chain();
-    if (!chain) return TEUK_EHIP;
-    std::lock_guard<std::mutex> turn(chain->lock);
-    if (chain->last) HIPCHK(hipStreamWaitEvent(st, chain->done, 0));
     HIPCHK(launch_init_res(g, d, st));
     int gate = 0;
     for (int done = 0; done < nsteps; done += kRing, gate ^= 1) {
       const int n = std::min(kRing, nsteps - done);
       if (has_src) HIPCHK(launch_source(g, d, 0, n, true, st));
-      HIPCHK(launch_resident(g, d, p->integrator, has_src, sh, ResSpan{0, p->N, 0, p->N, d.U, d.D, nullptr, 0}, n, nsteps,
-                             d.ctl->gate + gate, res_wait_ticks(kResWait), st));
+      rc = resident_launch(
+          st,
+          [&]() {
+            return launch_resident(g, d, p->integrator, has_src, sh, ResSpan{0, p->N, 0, p->N, d.U, d.D, nullptr, 0}, n,
+                                   nsteps, d.ctl->gate + gate, res_wait_ticks(kResWait), st);
+          },
+          false);
+      if (rc) return rc;
       HIPCHK(launch_finalize(g, d, n, d.ctl->gate + gate, d.ctl->gate + (gate ^ 1), st));
     }
     HIPCHK(hipStreamSynchronize(st));
-    chain->last = nullptr;   // (waited for above)
+    if (ResidentChain *chain = resident_chain()) {
+      std::lock_guard<std::mutex> hold_chain(chain->lock);
+      chain->unrecorded = false;   // (waited for above)
+    }
     HIPCHK(hipMemcpy(&c, d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
     if (c.fail && (rc = stage_chunks(nsteps - c.k))) return rc;
   } else if ((rc = stage_chunks(nsteps))) {
