@@ -176,20 +176,38 @@ struct ResidentChain {
 constexpr int kMaxDevices = 64;
 ResidentChain g_chain[kMaxDevices];
 
-// The current device's chain.
-ResidentChain *resident_chain() {
+// The chain of a stream's device (of the current one for the null stream).
+ResidentChain *resident_chain(hipStream_t stream, int *device = nullptr) {
   int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+  if ((stream ? hipStreamGetDevice(stream, &dev) : hipGetDevice(&dev)) != hipSuccess) return nullptr;
+  if (dev < 0 || dev >= kMaxDevices) return nullptr;
+  if (device) *device = dev;
   return &g_chain[dev];
 }
 
+// A device made current for a scope.
+struct OnDevice {
+  int was = -1;
+  bool ok;
+  explicit OnDevice(int device) {
+    ok = hipGetDevice(&was) == hipSuccess && (was == device || hipSetDevice(device) == hipSuccess);
+    if (was == device) was = -1;
+  }
+  ~OnDevice() {
+    if (was >= 0) (void)hipSetDevice(was);
+  }
+};
+
 template <class Launch>
 int resident_launch(hipStream_t stream, Launch launch, bool may_create = true) {
-  ResidentChain *chain = resident_chain();
+  int device = -1;
+  ResidentChain *chain = resident_chain(stream, &device);
   if (!chain) return TEUK_EHIP;
   ResidentChain &c = *chain;
   std::lock_guard<std::mutex> hold(c.lock);
   if (!c.done && may_create) {
+    const OnDevice on(device);   // events are recorded on streams of their own device only
+    if (!on.ok) return TEUK_EHIP;
     HIPCHK(hipEventCreateWithFlags(&c.done, hipEventDisableTiming));
     if (c.unrecorded) {
       HIPCHK(hipEventRecord(c.done, nullptr));
@@ -1807,7 +1825,7 @@ int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *th
       HIPCHK(launch_finalize(g, d, n, d.ctl->gate + gate, d.ctl->gate + (gate ^ 1), st));
     }
     HIPCHK(hipStreamSynchronize(st));
-    if (ResidentChain *chain = resident_chain()) {
+    if (ResidentChain *chain = resident_chain(st)) {
       std::lock_guard<std::mutex> hold_chain(chain->lock);
       chain->unrecorded = false;   // (waited for above)
     }

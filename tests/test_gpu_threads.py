@@ -57,3 +57,29 @@ def test_solvers_on_concurrent_host_threads():
         assert np.array_equal(u, u2)
         assert np.array_equal(h, h2)
         assert np.array_equal(psi, psi2)
+
+
+def test_solver_of_another_device_than_the_current_one():
+    """Steps and results of a solver made on the second device while the
+    first is current (its launches are ordered on its own device)."""
+    import ctypes
+    teuk.lib()
+    hip = ctypes.CDLL(next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l))
+    n = ctypes.c_int()
+    assert hip.hipGetDeviceCount(ctypes.byref(n)) == 0
+    if n.value < 2:
+        pytest.skip("needs two devices")
+    p, u0, _, steps = case(2, 1, 1)
+    with teuk.Solver(p) as s:
+        s.set_fields(u0)
+        s.step(steps)
+        s.sync()
+        want = s.get_fields()
+    assert hip.hipSetDevice(1) == 0
+    with teuk.Solver(p) as s:
+        s.set_fields(u0)
+        assert hip.hipSetDevice(0) == 0
+        for _ in range(3):
+            s.step(steps // 3)
+        s.sync()
+        assert np.array_equal(s.get_fields(), want)
