@@ -96,7 +96,7 @@ struct teuk_batch {
   BatchTile *d_tiles = nullptr;
   size_t tiles_cap = 0;
   // Resident launches for the members whose fields fit on the chip, until a
-  // launch shape is set for the stage kernels.
+  // launch shape is set for the stage kernels (and after, where asked for).
   bool resident = true;
   ResBlock *d_blocks = nullptr;
   size_t blocks_cap = 0;
@@ -1543,6 +1543,13 @@ int teuk_batch_set_tiling(teuk_batch *b, int waves_per_block, int waves_per_eu, 
   b->order = order;
   b->chunk = chunk;
   b->resident = false;
+  b->dirty = true;
+  return TEUK_OK;
+}
+
+int teuk_batch_set_resident(teuk_batch *b, int on) {
+  if (!b) return TEUK_EINVAL;
+  b->resident = on != 0;
   b->dirty = true;
   return TEUK_OK;
 }

@@ -191,10 +191,16 @@ class Server:
                 st["prepare_s"] += time.perf_counter() - ts
 
         batch = teuk.Batch(integrator=self.integrator, hbm_budget=self.hbm_budget)
-        # without a launch shape the members' fields stay on the chip
-        # between their steps (teuk_set_resident_wait in include/teuk.h)
         if self.tiling:
             batch.set_tiling(chunk=self.chunk, **self.tiling)
+        else:
+            # members that fit on the chip stay there between their steps;
+            # for the others 2-row wavefronts, 1 per block, built for 3 waves
+            # per SIMD, the fastest over a served window; us a stage of
+            # every member with it / without a shape: 8 x 1024x136 21.5 /
+            # 23.9, 4 x 4096x136 45.0 / 46.8, 16384x256 107.7 / 115.0,
+            # 2 x 32768x64 100.7 / 105.2, 2 x 512x256 10.4 / 9.9
+            batch.set_tiling(1, 3, 0, self.chunk, theta_rows=2, resident=True)
         try:
             while pending or queue or live:
                 if deadline is not None and now() >= deadline:

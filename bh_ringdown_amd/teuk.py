@@ -78,6 +78,7 @@ EXPORTS = [
     "teuk_source_coeffs", "teuk_source_patch", "teuk_grid_half", "teuk_create_staggered",
     "teuk_trajectory_schedule_staggered", "teuk_status", "teuk_solve_noalloc", "teuk_batch_set_cache_groups",
     "teuk_ot_transition", "teuk_set_resident_wait", "teuk_set_exchange_reads", "teuk_resident", "teuk_set_theta_rows", "teuk_batch_set_theta_rows",
+    "teuk_batch_set_resident",
 ]
 
 _lib = None
@@ -135,6 +136,7 @@ def lib():
         "teuk_set_resident_wait": ([vp, ctypes.c_double], ctypes.c_int),
         "teuk_set_exchange_reads": ([vp, ctypes.c_int], ctypes.c_int),
         "teuk_batch_set_theta_rows": ([vp, ctypes.c_int], ctypes.c_int),
+        "teuk_batch_set_resident": ([vp, ctypes.c_int], ctypes.c_int),
         "teuk_ot_transition": ([ctypes.c_double, _dp, _dp], ctypes.c_int),
         "teuk_remaining": ([vp, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
         "teuk_source_coeffs": ([vp, ctypes.c_int, ctypes.c_int, _dp], ctypes.c_int),
@@ -436,11 +438,15 @@ class Batch:
         _check(lib().teuk_batch_remove(self._h, solver._h), "teuk_batch_remove")
         self.members.remove(solver)
 
-    def set_tiling(self, waves_per_block=4, waves_per_eu=2, order=0, chunk=32, theta_rows=None):
+    def set_tiling(self, waves_per_block=4, waves_per_eu=2, order=0, chunk=32, theta_rows=None, resident=False):
+        """Launch shape of the stage kernels: for all members, or with
+        `resident` for those that do not fit on the chip."""
         _check(lib().teuk_batch_set_tiling(self._h, int(waves_per_block), int(waves_per_eu), int(order),
                                            int(chunk)), "teuk_batch_set_tiling")
         if theta_rows is not None:
             _check(lib().teuk_batch_set_theta_rows(self._h, int(theta_rows)), "teuk_batch_set_theta_rows")
+        if resident:
+            _check(lib().teuk_batch_set_resident(self._h, 1), "teuk_batch_set_resident")
 
     def set_cache_groups(self, group_bytes):
         """Step members in groups whose field state fits group_bytes (0 = one group)."""

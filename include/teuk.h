@@ -243,9 +243,11 @@ int teuk_remaining(teuk_solver *s, int *steps);
  * run.sh:3-16).  A batch steps many solvers together.  Members whose fields
  * fit on the chip share resident launches (teuk_set_resident_wait), as many
  * to a launch as the CUs hold, until a launch shape is set for the batch
- * (teuk_batch_set_tiling, teuk_batch_set_theta_rows).  For the others each RK
- * stage of every member is one launch (blocks index a table of {solver,
- * tile}); chunks of steps are captured in a hipGraph.  Members may differ in N, M, a, m, dt,
+ * (teuk_batch_set_tiling, teuk_batch_set_theta_rows; but see
+ * teuk_batch_set_resident).  For the others, also those that a solver alone
+ * steps in segments and so about twice as fast, each RK stage of every member
+ * is one launch (blocks index a table of {solver, tile}); chunks of steps are
+ * captured in a hipGraph.  Members may differ in N, M, a, m, dt,
  * source and length; each stops at its own schedule end.  A member's results
  * are bitwise those of stepping it alone.  Members must share the
  * integrator.  While in a batch a solver is stepped only by its batch;
@@ -265,8 +267,12 @@ int teuk_batch_set_tiling(teuk_batch *b, int waves_per_block, int waves_per_eu, 
 /* Theta rows per stage-kernel wavefront for every member (as
  * teuk_set_theta_rows). */
 int teuk_batch_set_theta_rows(teuk_batch *b, int rows);
-/* Cache groups: the unfinished members, in list order, are split into
- * groups whose field state (RK state planes and the dbdx plane, 136 B per
+/* on 1: members that fit on the chip share resident launches also where a
+ * launch shape was set, which is then the others'; 0: all by the stage
+ * kernels. */
+int teuk_batch_set_resident(teuk_batch *b, int on);
+/* Cache groups: the unfinished members that are stepped by the stage kernels,
+ * in list order, are split into groups whose field state (RK state planes and the dbdx plane, 136 B per
  * point for RK4) stays within group_bytes, so that a group's fields stay in
  * the last-level cache while it runs a chunk of steps; each chunk then runs
  * group after group.  0 (the default) = one group.  Results do not depend

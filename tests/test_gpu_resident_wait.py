@@ -78,6 +78,18 @@ def test_resident_of_members():
     assert [s.resident() for s in solvers] == [True, False, False]
     b.set_tiling(1, 2, 0, 32, theta_rows=2)
     assert not any(s.resident() for s in solvers)
+    b.set_tiling(1, 3, 0, 32, theta_rows=2, resident=True)      # the shape for those that do not fit
+    assert [s.resident() for s in solvers] == [True, False, False]
+    b.step(2)
+    b.sync()
+    assert teuk.lib().teuk_batch_set_resident(b._h, 0) == teuk.TEUK_OK
+    b.step(2)
+    b.sync()
+    assert not any(s.resident() for s in solvers)
+    for s, (p, u0, _) in zip(solvers, specs):
+        with start(p, u0, None, 8) as one:
+            one.step(8)
+            assert np.array_equal(s.get_fields(), one.get_fields())
     b.close()
     assert [s.resident() for s in solvers] == [True, True, False]      # alone again
     for s in solvers:

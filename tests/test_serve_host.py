@@ -273,3 +273,22 @@ def test_server_retires_a_stalled_solve_too(monkeypatch):
     Batch.code = teuk.TEUK_EHIP
     with pytest.raises(teuk.TeukError):
         serve.Server(hbm_budget=1 << 40, chunk=16, target_points=1 << 30).run(reqs)
+
+
+@pytest.mark.parametrize("tiling", [None, {"waves_per_block": 2, "waves_per_eu": 2, "theta_rows": 4}])
+def test_server_sets_its_batch_up(monkeypatch, tiling):
+    """Without a launch shape of the caller's the batch gets the server's, for
+    members that do not fit on the chip, and its chunk; with one, that."""
+    calls = []
+
+    class Batch(_FakeBatch):
+        def set_tiling(self, *a, **k):
+            names = ("waves_per_block", "waves_per_eu", "order", "chunk")
+            calls.append({**dict(zip(names, a)), **k})
+
+    monkeypatch.setattr(serve, "prepare_host", _fake_host)
+    monkeypatch.setattr(serve, "prepare_device", lambda p, req, th, rows: (p, _FakeSolver(p)))
+    monkeypatch.setattr(serve.teuk, "Batch", Batch)
+    serve.Server(hbm_budget=1 << 40, chunk=48, tiling=tiling).run([])
+    want = tiling or {"waves_per_block": 1, "waves_per_eu": 3, "order": 0, "theta_rows": 2, "resident": True}
+    assert calls == [{**want, "chunk": 48}]
