@@ -283,8 +283,8 @@ hipError_t timing_begin(teuk_solver *s, int stages) {
         const hipError_t err = hipEventCreate(&e);
         if (err != hipSuccess) return err;
         s->ev.push_back(e);
+        s->ev_stages.resize((s->ev.size() + 1) / 2);
       }
-      s->ev_stages.resize(s->ev.size() / 2);
     } else {
       flush_timing(s);
     }
@@ -307,14 +307,15 @@ int enqueue_step(teuk_solver *s, int k_rel) {
   // half steps for the staggered scheme)
   const int group = s->g.stag ? kRing / 2 : kRing;
   if (s->has_src && k_rel % group == 0) HIPCHK(launch_source(s->g, s->d, k_rel, kRing, false, run_stream(s)));
-  if (s->timing) HIPCHK(timing_begin(s, nstage));
+  const bool timed = s->timing && !s->batch;   // (the events are on the solver's own stream)
+  if (timed) HIPCHK(timing_begin(s, nstage));
   if (s->g.stag) {
     HIPCHK(launch_so2_step(s->g, s->d, s->has_src, k_rel, run_stream(s)));
   } else {
     for (int st = 1; st <= nstage; st++)
       HIPCHK(launch_stage(s->g, s->d, s->P.integrator, st, s->has_src, k_rel, s->tiling, run_stream(s)));
   }
-  if (s->timing) HIPCHK(timing_end(s));
+  if (timed) HIPCHK(timing_end(s));
   return TEUK_OK;
 }
 
@@ -393,6 +394,7 @@ int read_ctl(teuk_solver *s, Ctl &c) {
     const int zero = 0;
     HIPCHK(hipMemcpy(&s->d.ctl->fail, &zero, sizeof zero, hipMemcpyHostToDevice));
     s->resident = false;
+    s->ev_used = 0;   // not timed: launches that took no step are among these
     for (const teuk_solver::Place &p : s->places)
       if (p.k == c.k) {   // where the first launch that gave up left the state
         s->d.U = p.U;

@@ -173,7 +173,8 @@ int teuk_read_psi(teuk_solver *s, int first, int max, double *psi, int *n);
 /* Kernel timing: when enabled, teuk_step brackets each step's back-to-back
  * stage-kernel launches (or each resident launch, of up to 32 steps) with a
  * pair of HIP events on the solver stream.  teuk_timing returns the number of
- * timed stages and their summed duration in milliseconds. */
+ * timed stages and their summed duration in milliseconds (without those of a
+ * resident launch that gave up, and of the ones waited for together with it). */
 int teuk_enable_timing(teuk_solver *s, int on);
 int teuk_timing(teuk_solver *s, long long *launches, double *ms);
 

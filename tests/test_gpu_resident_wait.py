@@ -94,3 +94,25 @@ def test_resident_of_members():
     assert [s.resident() for s in solvers] == [True, True, False]      # alone again
     for s in solvers:
         s.close()
+
+
+def test_launches_that_gave_up_are_not_timed():
+    p, u0, _ = setup(1024, 32, 1, 2, 96)
+    with start(p, u0, None, 96) as s:
+        s.enable_timing(True)
+        s.step(32)
+        s.sync()
+        assert s.timing()[0] == 4 * 32
+        s.set_resident_wait(0.0)
+        s.step(64)              # two launches that change nothing
+        s.sync()
+        n, ms = s.timing()
+        assert n == 4 * 96 and 0.0 < ms < 100.0
+    b, solvers = batch_of([setup(1024, 32, 1, 2, 32)], 32)
+    solvers[0].enable_timing(True)      # a batch's steps are not a solver's own
+    solvers[0].set_resident_wait(0.0)
+    b.step(32)
+    b.sync()
+    assert solvers[0].timing()[0] == 0 and solvers[0].progress()[0] == 32
+    b.close()
+    solvers[0].close()
