@@ -24,9 +24,12 @@ tune_batch() times whole batch steps.  Winners are kept in a JSON cache
 grid shape and integrator, and looked up by best_solver_tiling() /
 best_batch_tiling() / best_batch_groups().
 
-The shapes are those of the per-stage kernels, which step grids of more than
-128 theta rows.  Setting one on a smaller grid's solver or batch takes it off
-resident stepping, which is the faster there.
+The shapes are those of the per-stage kernels, and setting one takes a solver
+or a batch off resident stepping, which is about twice as fast.  So the
+library's own choice (no shape set) is timed too, and where it wins no shape
+is returned.  The committed table has no such times: its entries are for
+solvers and batches that are kept off resident stepping; ask
+Solver.resident() first.
 """
 import itertools
 import json
@@ -88,13 +91,15 @@ def _probe_params(N, M, integrator, steps):
 
 
 def tune_solver(N, M, integrator=1, steps=60, repeats=2, store=True, rows=(2, 4, 8)):
-    """Time every (waves_per_block, waves_per_eu, theta_rows) on an N x M
-    grid; returns (best, {candidate: us per stage launch})."""
+    """Time the library's own choice (None) and every (waves_per_block,
+    waves_per_eu, theta_rows) on an N x M grid; returns (best, {candidate: us
+    per stage})."""
     times = {}
-    for wpb, wpe, tr in itertools.product((1, 2, 4), (2, 3, 4), rows):
+    for shape in (None, *itertools.product((1, 2, 4), (2, 3, 4), rows)):
         p = _probe_params(N, M, integrator, steps * repeats + 10)
         with teuk.Solver(p) as s:
-            s.set_tiling(wpb, wpe, tr)
+            if shape:
+                s.set_tiling(*shape)
             s.step(5)
             s.sync()
             s.enable_timing(True)
@@ -102,11 +107,12 @@ def tune_solver(N, M, integrator=1, steps=60, repeats=2, store=True, rows=(2, 4,
                 s.step(steps)
             s.sync()
             n, ms = s.timing()
-        times[(wpb, wpe, tr)] = 1e3 * ms / n
+        times[shape] = 1e3 * ms / n
     best = min(times, key=times.get)
     if store:
-        _store(solver_key(N, M, integrator), {"waves_per_block": best[0], "waves_per_eu": best[1],
-                                              "theta_rows": best[2], "us_per_launch": times[best]})
+        top = min(filter(None, times), key=times.get)
+        _store(solver_key(N, M, integrator), {"waves_per_block": top[0], "waves_per_eu": top[1], "theta_rows": top[2],
+                                              "us_per_launch": times[top], "default_us": times[None]})
     return best, times
 
 
@@ -119,46 +125,58 @@ def tune_batch(shapes, integrator=1, steps=64, store=True, chunks=(16, 32, 64), 
                rows=(2, 4, 8), wpes=(2, 3)):
     """Time whole batch steps of probe solvers of the given (N, M) shapes
     (one probe per entry, so repeat a shape to tune a batch of many) for
-    every (waves_per_block, waves_per_eu, order, chunk, cache-group bytes,
-    theta_rows); returns (best, {candidate: seconds per step})."""
+    the library's own choice (None) and every (waves_per_block, waves_per_eu,
+    order, chunk, cache-group bytes, theta_rows); returns (best, {candidate:
+    seconds per step})."""
     times = {}
-    for wpb, wpe, order, chunk, gb, tr in itertools.product((1, 2, 4), wpes, (0, 1), chunks, group_bytes, rows):
+    for sched in (None, *itertools.product((1, 2, 4), wpes, (0, 1), chunks, group_bytes, rows)):
         solvers = [teuk.Solver(_probe_params(n, m, integrator, 3 * steps + 10)) for n, m in shapes]
         try:
             with teuk.Batch(integrator=integrator) as b:
-                b.set_tiling(wpb, wpe, order, chunk, tr)
-                b.set_cache_groups(gb)
+                if sched:
+                    b.set_tiling(*sched[:4], sched[5])
+                    b.set_cache_groups(sched[4])
                 for s in solvers:
                     b.add(s)
-                b.step(chunk)
+                b.step(sched[3] if sched else steps)
                 b.sync()
                 t0 = time.perf_counter()
                 b.step(2 * steps)
                 b.sync()
-                times[(wpb, wpe, order, chunk, gb, tr)] = (time.perf_counter() - t0) / (2 * steps)
+                times[sched] = (time.perf_counter() - t0) / (2 * steps)
         finally:
             for s in solvers:
                 s.close()
     best = min(times, key=times.get)
     if store:
-        _store(batch_key(shapes, integrator), {"waves_per_block": best[0], "waves_per_eu": best[1],
-                                               "order": best[2], "chunk": best[3], "group_bytes": best[4],
-                                               "theta_rows": best[5], "s_per_step": times[best]})
+        top = min(filter(None, times), key=times.get)
+        _store(batch_key(shapes, integrator), {"waves_per_block": top[0], "waves_per_eu": top[1], "order": top[2],
+                                               "chunk": top[3], "group_bytes": top[4], "theta_rows": top[5],
+                                               "s_per_step": times[top], "default_s": times[None]})
     return best, times
+
+
+def _beaten(e):
+    """Whether the library's own choice was as fast as the entry's shape."""
+    return (e.get("default_us", float("inf")) <= e.get("us_per_launch", 0.0)
+            or e.get("default_s", float("inf")) <= e.get("s_per_step", 0.0))
 
 
 def best_solver_tiling(N, M, integrator=1):
     """Tuned launch shape for a grid as Solver.set_tiling keyword arguments,
-    or None."""
+    or None where there is none or the library's own choice is the faster.
+    It is for a solver whose resident() is false: setting it ends resident
+    stepping."""
     e = _load().get(solver_key(N, M, integrator))
-    if not e:
+    if not e or _beaten(e):
         return None
     return {"waves_per_block": e["waves_per_block"], "waves_per_eu": e["waves_per_eu"],
             "theta_rows": e.get("theta_rows", 8)}
 
 
 def best_batch_tiling(shapes, integrator=1):
-    """Tuned batch schedule as set_tiling keyword arguments, or None.  Falls
+    """Tuned batch schedule as set_tiling keyword arguments, or None (also
+    where the library's own choice is the faster).  Falls
     back to the entry for the same set of shapes (any counts), then to one
     for the same set of row counts M, if the exact batch was not tuned."""
     data = _load()
@@ -173,7 +191,7 @@ def best_batch_tiling(shapes, integrator=1):
         if e is None:
             ms = {m for _, m in shapes}
             e = next((v for k, v in cands if {m for _, m in kshapes(k)} == ms), None)
-    if not e:
+    if not e or _beaten(e):
         return None
     return {"waves_per_block": e["waves_per_block"], "waves_per_eu": e["waves_per_eu"], "order": e["order"],
             "chunk": e["chunk"], "theta_rows": e.get("theta_rows", 8)}
@@ -183,7 +201,11 @@ def best_batch_groups(shapes, integrator=1):
     """Tuned cache-group bytes for a batch (0 = off, also when not tuned)."""
     data = _load()
     e = data.get(batch_key(shapes, integrator))
-    return int(e.get("group_bytes", 0)) if e else 0
+    return int(e.get("group_bytes", 0)) if e and not _beaten(e) else 0
+
+
+def _name(candidate):
+    return ",".join(map(str, candidate)) if candidate else "default"
 
 
 def main(argv=None):
@@ -198,7 +220,7 @@ def main(argv=None):
     for s in args.solver:
         N, M = map(int, s.split("x"))
         best, t = tune_solver(N, M, args.integrator)
-        print(json.dumps({"solver": s, "best": best, "us": {",".join(map(str, k)): round(v, 3) for k, v in t.items()}}),
+        print(json.dumps({"solver": s, "best": best, "us": {_name(k): round(v, 3) for k, v in t.items()}}),
               flush=True)
     for spec in args.batch:
         shapes = []
@@ -207,7 +229,7 @@ def main(argv=None):
             shapes += [tuple(map(int, sh.split("x")))] * int(cnt or 1)
         best, t = tune_batch(shapes, args.integrator, chunks=tuple(int(c) for c in args.chunks.split(",")))
         print(json.dumps({"batch": spec, "best": best,
-                          "ms_per_step": {",".join(map(str, k)): round(1e3 * v, 4) for k, v in t.items()}}),
+                          "ms_per_step": {_name(k): round(1e3 * v, 4) for k, v in t.items()}}),
               flush=True)
     return 0
 
