@@ -1737,7 +1737,14 @@ size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *theta, const double *u0,
                        const teuk_source_step *steps, int nsteps, double *u_out, teuk_output_row *rows,
                        int max_rows, int *nrows) {
+  return teuk_solve_noalloc_wait(p, r_c, theta, u0, steps, nsteps, u_out, rows, max_rows, nrows, kResWait);
+}
+
+int teuk_solve_noalloc_wait(const teuk_params *p, const double *r_c, const double *theta, const double *u0,
+                            const teuk_source_step *steps, int nsteps, double *u_out, teuk_output_row *rows,
+                            int max_rows, int *nrows, double wait) {
   if (nrows) *nrows = 0;
+  if (!(wait >= 0.0)) return TEUK_EINVAL;
   if (!p || !r_c || !theta || nsteps < 0 || max_rows < 0 || (max_rows > 0 && !rows)) return TEUK_EINVAL;
   int rc = validate(p);
   if (rc) return rc;
@@ -1827,7 +1834,7 @@ int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *th
           st,
           [&]() {
             return launch_resident(g, d, p->integrator, has_src, sh, ResSpan{0, p->N, 0, p->N, d.U, d.D, nullptr, 0}, n,
-                                   nsteps, d.ctl->gate + gate, res_wait_ticks(kResWait), st);
+                                   nsteps, d.ctl->gate + gate, res_wait_ticks(wait), st);
           },
           false);
       if (rc) return rc;

@@ -78,7 +78,7 @@ EXPORTS = [
     "teuk_source_coeffs", "teuk_source_patch", "teuk_grid_half", "teuk_create_staggered",
     "teuk_trajectory_schedule_staggered", "teuk_status", "teuk_solve_noalloc", "teuk_batch_set_cache_groups",
     "teuk_ot_transition", "teuk_set_resident_wait", "teuk_set_exchange_reads", "teuk_resident", "teuk_set_theta_rows", "teuk_batch_set_theta_rows",
-    "teuk_batch_set_resident",
+    "teuk_batch_set_resident", "teuk_solve_noalloc_wait",
 ]
 
 _lib = None
@@ -115,6 +115,9 @@ def lib():
         "teuk_status": ([vp], ctypes.c_int),
         "teuk_solve_noalloc": ([P, _dp, _dp, _dp, ctypes.POINTER(SourceStep), ctypes.c_int, _dp,
                                 ctypes.POINTER(OutputRow), ctypes.c_int, ctypes.POINTER(ctypes.c_int)],
+                               ctypes.c_int),
+        "teuk_solve_noalloc_wait": ([P, _dp, _dp, _dp, ctypes.POINTER(SourceStep), ctypes.c_int, _dp,
+                                ctypes.POINTER(OutputRow), ctypes.c_int, ctypes.POINTER(ctypes.c_int), ctypes.c_double],
                                ctypes.c_int),
         "teuk_progress": ([vp, ctypes.POINTER(ctypes.c_int), _dp], ctypes.c_int),
         "teuk_read_output": ([vp, ctypes.c_int, ctypes.c_int, ctypes.POINTER(OutputRow),
@@ -464,8 +467,9 @@ class Batch:
         return {"members": m.value, "active": a.value, "bytes": b.value}
 
 
-def solve_noalloc(p, r_c, theta, nsteps, u0=None, steps=None, max_rows=None):
-    """teuk_solve_noalloc: a whole solve in the library's fixed scratch memory.
+def solve_noalloc(p, r_c, theta, nsteps, u0=None, steps=None, max_rows=None, wait=None):
+    """teuk_solve_noalloc: a whole solve in the library's fixed scratch memory
+    (teuk_solve_noalloc_wait where a wait is given, in seconds).
     Returns (code, fields[4, M, N], records as Solver.output()); code is
     TEUK_OK, TEUK_EDIVERGED, TEUK_ESTALLED or TEUK_ETOOBIG (then fields and
     records are empty); other errors raise."""
@@ -484,8 +488,9 @@ def solve_noalloc(p, r_c, theta, nsteps, u0=None, steps=None, max_rows=None):
     rows = (OutputRow * max(cap, 1))()
     u = np.zeros((4, p.M, p.N))
     n = ctypes.c_int()
-    rc = lib().teuk_solve_noalloc(ctypes.byref(p), _ptr(r_c), _ptr(theta), u0p, arr, int(nsteps), _ptr(u), rows,
-                                  cap, ctypes.byref(n))
+    args = (ctypes.byref(p), _ptr(r_c), _ptr(theta), u0p, arr, int(nsteps), _ptr(u), rows, cap, ctypes.byref(n))
+    rc = (lib().teuk_solve_noalloc(*args) if wait is None
+          else lib().teuk_solve_noalloc_wait(*args, float(wait)))
     if rc not in (TEUK_OK, TEUK_EDIVERGED, TEUK_ESTALLED, TEUK_ETOOBIG):
         _check(rc, "teuk_solve_noalloc")
     k = n.value

@@ -338,6 +338,11 @@ int teuk_traj_plunge(double a, double eta, double iota, double r0_over_isco, dou
 int teuk_solve_noalloc(const teuk_params *p, const double *r_c, const double *theta,
                        const double *u0, const teuk_source_step *steps, int nsteps,
                        double *u_out, teuk_output_row *rows, int max_rows, int *nrows);
+/* The same with the wait of its resident launches given (see
+ * teuk_set_resident_wait); teuk_solve_noalloc waits 0.25 s. */
+int teuk_solve_noalloc_wait(const teuk_params *p, const double *r_c, const double *theta,
+                            const double *u0, const teuk_source_step *steps, int nsteps,
+                            double *u_out, teuk_output_row *rows, int max_rows, int *nrows, double wait);
 
 /* The universal Ori-Thorne transition function X(L) (X'' = -X^2 - L,
  * X -> sqrt(-L) as L -> -inf) and X'(L), for -40 <= L <= 3.4, as
