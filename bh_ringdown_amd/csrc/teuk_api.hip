@@ -789,8 +789,9 @@ void bind_layout(const teuk_params *p, const Layout &L, char *base, DevState &d)
 }
 
 // A state that holds nothing between steps: every scheme writes it before it
-// reads it.  (d.C of the Runge-Kutta schemes holds what resident stepping in
-// segments prepares once.)
+// reads it.  (The staggered scheme has no d.D; its half-point fields d.C are
+// formed anew each step, as are the exchange slots and coefficient values that
+// resident launches keep in d.C.)
 double *stage_state(const DevState &d) { return d.D ? d.D : d.C; }
 
 // The run description of a solve.

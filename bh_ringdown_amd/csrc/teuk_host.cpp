@@ -273,6 +273,9 @@ bool resident_shape(int N, int M, int cus, ResShape &sh) {
 }
 
 // Measured time of one stage with tiles of kResCP[c] columns per thread (us).
+// Columns of 72 to 128 rows take 5.8, 7.9 and 9.5 with 4, 6 and 8, 5 to 8 %
+// more than 64 rows' (there are no tiles of 1 or 2): which width is the
+// cheapest does not change by it.
 static double stage_us(int M, int c) {
   static const double k32[5] = {2.5, 2.9, 5.2, 7.2, 8.9}, k64[5] = {3.2, 3.5, 5.4, 7.6, 8.9};
   return M <= 32 ? k32[c] : k64[c];
@@ -364,7 +367,9 @@ std::vector<ResGroup> resident_groups(const std::vector<std::pair<int, int>> &sh
 // columns beside them that the steps reach (H on each inner side), so fewer
 // steps mean less to compute twice and more launches, each about 25 us of
 // loads, stores and set-up.  The per-stage kernels take about 19.5 us a stage
-// and million points; the plan must beat that by a tenth.
+// and million points (16 to 23 over 12288x72 ... 65536x96); the plan must beat
+// that by a tenth (16384x96: 23.5 us a stage in segments, 25.1 by stages;
+// 16384x72, by stages: 20.3).
 ResSegments resident_segments(int N, int M, int integrator, int cus) {
   ResSegments best;
   ResShape whole;

@@ -358,11 +358,11 @@ hipError_t launch_stage(const Grid &g, const DevState &d, int integrator, int st
 // pair, or all `others` of it, is cleared), or null.
 hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, hipStream_t s,
                            int others = 1);
-// Flags and column constants of resident stepping, into the set-up plane.
 // The ABI's four real planes to the device's two planes of pairs and back
 // (in and out apart).
 hipError_t launch_fields_join(const double *in, double *out, size_t NM, hipStream_t s);
 hipError_t launch_fields_split(const double *in, double *out, size_t NM, hipStream_t s);
+// Flags and column constants of resident stepping, into the set-up plane.
 hipError_t launch_init_res(const Grid &g, const DevState &d, hipStream_t s);
 // nsteps <= kRing steps of one solve (at most to step nt) in one launch.
 hipError_t launch_resident(const Grid &g, const DevState &d, int integrator, bool has_src, ResShape sh,

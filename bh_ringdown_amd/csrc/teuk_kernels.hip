@@ -302,7 +302,10 @@ Tiling default_tiling(int N, int M) {
   // grids 8-row chunks, which re-read the fewest halo rows, win (2-row / 8-row,
   // us a stage: 16000 x 256 SSP-RK3 91.2 / 85.0, RK4 99.6 / 94.7; 24576 x 192
   // 105.2 / 100.0; 8192 x 512 93.2 / 88.7), not on lower ones (32768 x 136 95.0
-  // / 99.5) nor below (12288 x 256, 3.1 M points, 59.3 / 61.2).
+  // / 99.5) nor below (12288 x 256, 3.1 M points, 59.3 / 61.2).  Above, 4-row
+  // chunks (4-row / 8-row, RK4: 32768 x 256 194.0 / 200.4, 45056 x 192 188.0 /
+  // 189.3, 65536 x 136 197.4 / 204.3), but for 512 rows and more, which are not
+  // told apart here (16384 x 512 207.2 / 196.9, 8192 x 1024 204.2 / 197.6).
   if (!large && (long long)N * M >= 7 * (1LL << 19) && M >= 192) return Tiling{1, 2, 8};
   t.rows = large ? 4 : kDefaultThetaRows;
   t.wpe = (!large && M >= 64) ? 3 : 2;
