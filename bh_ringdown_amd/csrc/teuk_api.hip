@@ -2,7 +2,11 @@
 // hipGraph-captured steps, trajectory consumption and the body() drop-in.
 #include <hip/hip_runtime.h>
 
+#include <unistd.h>
+
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -27,21 +31,17 @@ struct teuk_solver {
   DevState d;
   Tiling tiling;
   // Resident stepping (teuk_resident.inc), unless the grid does not fit on
-  // the chip, a launch shape was set for the stage kernels, or a launch gave up.
+  // the chip, a launch shape was set for the stage kernels, or launches waited
+  // too long in a row.
   bool resident = false;
   ResShape res_shape{0, 0, 0};
-  double res_wait = kResWait;
+  double res_wait = kResWait, res_patience = kResPatience;
+  int asides = 0;                // launches that had stepped aside when the control block was last read
   int gate = 0;                  // which of the control block's two gates is next
   bool res_pending = false;      // resident launches since the control block was last read
   // Grids beyond the chip: stepped in segments (resident_segments), from the
-  // state U into D, which then change places.  The places at the start of
-  // each chunk since the control block was last read, by step.
+  // state U into D and back (ResTries::cur).
   ResSegments segs;
-  struct Place {
-    int k;
-    double *U, *D;
-  };
-  std::vector<Place> places;
   teuk_batch *batch = nullptr;   // set while a batch drives this solver
   hipStream_t stream = nullptr;
   int nt = 0;              // scheduled steps: (int)(T/dt), body.cu:59
@@ -88,7 +88,7 @@ struct teuk_batch {
     int CP = 0, MT = 0;
     size_t block_off = 0, lds = 0;
     int nblocks = 0;
-    double wait = 0.0;
+    double wait = 0.0, patience = 0.0;
   };
   std::vector<Group> groups;
   SolveDesc *d_desc = nullptr;
@@ -327,14 +327,33 @@ int stage_steps(teuk_solver *s, int n) {
     if (rc) return rc;
   }
   HIPCHK(launch_sentinel(s->g, s->d, run_stream(s)));
-  HIPCHK(launch_finalize(s->g, s->d, n, nullptr, nullptr, run_stream(s)));
+  HIPCHK(launch_finalize(s->g, s->d, n, nullptr, nullptr, ResTry{}, run_stream(s)));
   return TEUK_OK;
+}
+
+// How long a launch waits, given the longest wait in a row and its first (s).
+ResTry res_try(double wait, double patience, bool flip) {
+  // a sequence of its own in each process (splitmix64)
+  static std::atomic<unsigned long long> next{(unsigned long long)getpid() * 0x9e3779b97f4a7c15ull ^
+                                              (unsigned long long)std::chrono::steady_clock::now().time_since_epoch().count()};
+  unsigned long long z = next.fetch_add(0x9e3779b97f4a7c15ull) + 0x9e3779b97f4a7c15ull;
+  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+  const double u = (double)((z ^ (z >> 31)) >> 11) * 0x1p-53;
+  ResTry t;
+  t.budget = res_wait_ticks(wait);
+  t.limit = std::min(t.budget, (long long)(std::min(patience * (0.5 + u), kResWaitMost) * 1e8));
+  t.flip = flip ? 1 : 0;
+  return t;
 }
 
 // n steps by resident launches of up to kRing steps each: the source patches
 // of its steps, the steps (with the sentinel's check of the last fields), the
-// records.
+// records.  (On the stream of the solver's batch where one's steps are caught
+// up with.)
 int resident_steps(teuk_solver *s, int n) {
+  const hipStream_t stream = run_stream(s);
+  const bool timed = s->timing && !s->batch;
   const bool whole = s->segs.spans.empty();
   const int most = whole ? kRing : s->segs.steps;
   for (int done = 0; done < n;) {
@@ -343,12 +362,13 @@ int resident_steps(teuk_solver *s, int n) {
     const int sets = whole ? 1 : kMaxSegments;
     ResGate *gates = whole ? s->d.ctl->gate : res_gates(s->d, s->P.N);
     ResGate *mine = gates + s->gate * sets, *other = gates + (s->gate ^ 1) * sets;
-    if (s->has_src) HIPCHK(launch_source(s->g, s->d, 0, m, true, s->stream));
-    if (s->timing) HIPCHK(timing_begin(s, m * stages_per_step(s->P.integrator)));
+    ResTry t;
+    if (s->has_src) HIPCHK(launch_source(s->g, s->d, 0, m, true, stream));
+    if (timed) HIPCHK(timing_begin(s, m * stages_per_step(s->P.integrator)));
     auto launch = [&](const ResShape &sh, const ResSpan &sp, ResGate *gate) {
-      return resident_launch(s->stream, [&]() {
-        return launch_resident(s->g, s->d, s->P.integrator, s->has_src, sh, sp, m, s->nt, gate,
-                               res_wait_ticks(s->res_wait), s->stream);
+      t = res_try(s->res_wait, s->res_patience, !whole);
+      return resident_launch(stream, [&]() {
+        return launch_resident(s->g, s->d, s->P.integrator, s->has_src, sh, sp, m, s->nt, gate, t.limit, stream);
       });
     };
     int rc = TEUK_OK;
@@ -357,8 +377,7 @@ int resident_steps(teuk_solver *s, int n) {
       rc = launch(s->res_shape, ResSpan{0, s->P.N, 0, s->P.N, s->d.U, s->d.D, nullptr, 0}, mine);
     } else {
       // The segment with the extraction column goes last: its time integrals
-      // are in place, and must not have moved if another launch gives up.
-      s->places.push_back({s->k_host + done, s->d.U, s->d.D});
+      // are in place, and must not have moved if another launch steps aside.
       used = (int)s->segs.spans.size();
       std::vector<ResSpan> order = s->segs.spans;
       std::stable_partition(order.begin(), order.end(),
@@ -374,9 +393,8 @@ int resident_steps(teuk_solver *s, int n) {
       }
     }
     if (rc) return rc;
-    if (s->timing) HIPCHK(timing_end(s));
-    HIPCHK(launch_finalize(s->g, s->d, m, mine + used - 1, other, s->stream, used));
-    if (!whole) std::swap(s->d.U, s->d.D);
+    if (timed) HIPCHK(timing_end(s));
+    HIPCHK(launch_finalize(s->g, s->d, m, mine + used - 1, other, t, stream, used));
     s->gate ^= 1;
     s->res_pending = true;
     done += m;
@@ -384,36 +402,37 @@ int resident_steps(teuk_solver *s, int n) {
   return TEUK_OK;
 }
 
-// The control block after everything queued for the solver.  Steps that a
-// resident launch did not take (it could not get all its blocks onto the GPU
-// in time) are run by the per-stage launches first.
+// The control block after everything queued for the solver.  Steps that are
+// missing as resident launches stepped aside are queued again first, by the
+// stage kernels where the launches had waited too long.
 int read_ctl(teuk_solver *s, Ctl &c) {
-  HIPCHK(hipStreamSynchronize(run_stream(s)));
-  HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
-  if (c.fail) {
-    const int zero = 0;
-    HIPCHK(hipMemcpy(&s->d.ctl->fail, &zero, sizeof zero, hipMemcpyHostToDevice));
-    s->resident = false;
-    s->ev_used = 0;   // not timed: launches that took no step are among these
-    for (const teuk_solver::Place &p : s->places)
-      if (p.k == c.k) {   // where the first launch that gave up left the state
-        s->d.U = p.U;
-        s->d.D = p.D;
-        break;
-      }
-    if (s->batch) s->batch->dirty = true;
-    int missing = s->k_host - c.k;
-    while (missing > 0) {
-      const int m = std::min(kRing, missing);
-      const int rc = stage_steps(s, m);
-      if (rc) return rc;
-      missing -= m;
-    }
+  for (;;) {
     HIPCHK(hipStreamSynchronize(run_stream(s)));
     HIPCHK(hipMemcpy(&c, s->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+    if (!s->res_pending) return TEUK_OK;
+    if (c.tries.asides != s->asides) {
+      s->asides = c.tries.asides;
+      s->ev_used = 0;   // not timed: launches that took no step are among these
+    }
+    if (c.tries.fail || c.tries.cur) {
+      if (c.tries.cur) std::swap(s->d.U, s->d.D);
+      if (c.tries.fail) {
+        s->resident = false;
+        if (s->batch) s->batch->dirty = true;
+      }
+      const ResTries none{0, 0, 0, 0, c.tries.asides};
+      HIPCHK(hipMemcpy(&s->d.ctl->tries, &none, sizeof none, hipMemcpyHostToDevice));
+    }
+    const int missing = s->k_host - c.k;
+    if (missing <= 0) break;
+    if (s->resident) {
+      if (const int rc = resident_steps(s, missing)) return rc;
+    } else {
+      for (int left = missing; left > 0; left -= kRing)
+        if (const int rc = stage_steps(s, std::min(kRing, left))) return rc;
+    }
   }
   s->res_pending = false;
-  s->places.clear();
   return TEUK_OK;
 }
 
@@ -434,7 +453,8 @@ int build_graph(teuk_solver *s, int steps) {
   int rc = TEUK_OK;
   for (int i = 0; i < steps && rc == TEUK_OK; i++) rc = enqueue_step(s, i);
   if (rc == TEUK_OK && launch_sentinel(s->g, s->d, s->stream) != hipSuccess) rc = TEUK_EHIP;
-  if (rc == TEUK_OK && launch_finalize(s->g, s->d, steps, nullptr, nullptr, s->stream) != hipSuccess) rc = TEUK_EHIP;
+  if (rc == TEUK_OK && launch_finalize(s->g, s->d, steps, nullptr, nullptr, ResTry{}, s->stream) != hipSuccess)
+    rc = TEUK_EHIP;
   hipError_t e = hipStreamEndCapture(s->stream, &graph);
   if (rc != TEUK_OK) {
     if (graph) (void)hipGraphDestroy(graph);
@@ -1120,6 +1140,7 @@ int teuk_enable_timing(teuk_solver *s, int on) {
 
 int teuk_timing(teuk_solver *s, long long *launches, double *ms) {
   if (!s) return TEUK_EINVAL;
+  if (const int rc = settle(s)) return rc;   // launches that stepped aside are not counted
   flush_timing(s);
   if (launches) *launches = s->timed_launches;
   if (ms) *ms = s->timed_ms;
@@ -1242,6 +1263,13 @@ int teuk_set_resident_wait(teuk_solver *s, double seconds) {
   return TEUK_OK;
 }
 
+int teuk_set_resident_patience(teuk_solver *s, double seconds) {
+  if (!s || !(seconds >= 0.0)) return TEUK_EINVAL;
+  s->res_patience = seconds;
+  if (s->batch) s->batch->dirty = true;
+  return TEUK_OK;
+}
+
 int teuk_set_exchange_reads(teuk_solver *s, int reads) {
   if (!s || reads < 0) return TEUK_EINVAL;
   if (const int rc = settle(s)) return rc;
@@ -1330,19 +1358,21 @@ int batch_rebuild(teuk_batch *b) {
     g.CP = rg.CP;
     g.MT = rg.MT;
     g.block_off = blocks.size();
-    std::vector<double> waits;
+    std::vector<double> waits, patiences;
     for (size_t m = 0; m < rg.members.size(); m++) {
       teuk_solver *s = fit[rg.members[m]];
       const int C = rg.C[m];
       if (s->has_src) g.max_cells = std::max(g.max_cells, s->P.ptsx * s->P.ptsy);
       g.lds = std::max(g.lds, res_lds_bytes(s->P.M, C, rg.CP));
       waits.push_back(s->res_wait);
+      patiences.push_back(s->res_patience);
       const int B = (s->P.N + C - 1) / C;
       for (int k = 0; k < B; k++) blocks.push_back(ResBlock{(int)hd.size() - g.first, k, C, B});
       hd.push_back(describe(s));
     }
     g.nblocks = (int)(blocks.size() - g.block_off);
     g.wait = res_shared_wait(waits);
+    g.patience = res_shared_wait(patiences);
     b->groups.push_back(g);
   }
   const size_t first_stage = b->groups.size();
@@ -1456,7 +1486,7 @@ int batch_enqueue(teuk_batch *b, const teuk_batch::Group &g, int nsteps) {
       HIPCHK(launch_stage_batch(tiles, g.ntiles, b->integrator, st, k, b->tiling, b->stream));
   }
   HIPCHK(launch_sentinel_batch(descs, g.count, b->stream));
-  HIPCHK(launch_finalize_batch(descs, g.count, nsteps, nullptr, nullptr, b->stream));
+  HIPCHK(launch_finalize_batch(descs, g.count, nsteps, nullptr, nullptr, ResTry{}, b->stream));
   return TEUK_OK;
 }
 
@@ -1467,12 +1497,13 @@ int batch_resident(teuk_batch *b, const teuk_batch::Group &g, int nsteps) {
     const int m = std::min(kRing, nsteps - done);
     if (g.max_cells > 0) HIPCHK(launch_source_batch(descs, g.count, g.max_cells, 0, m, true, b->stream));
     ResGate *gate = b->gates + b->gate, *other = b->gates + (b->gate ^ 1);
+    const ResTry t = res_try(g.wait, g.patience, false);
     const int rc = resident_launch(b->stream, [&]() {
       return launch_resident_batch(descs, b->d_blocks + g.block_off, g.nblocks, b->integrator, g.CP, g.MT, g.lds, m,
-                                   gate, res_wait_ticks(g.wait), b->stream);
+                                   gate, t.limit, b->stream);
     });
     if (rc) return rc;
-    HIPCHK(launch_finalize_batch(descs, g.count, m, gate, other, b->stream));
+    HIPCHK(launch_finalize_batch(descs, g.count, m, gate, other, t, b->stream));
     b->gate ^= 1;
     done += m;
   }
@@ -1819,7 +1850,7 @@ int teuk_solve_noalloc_wait(const teuk_params *p, const double *r_c, const doubl
         for (int s = 1; s <= nstage; s++) HIPCHK(launch_stage(g, d, p->integrator, s, has_src, i, tiling, st));
       }
       HIPCHK(launch_sentinel(g, d, st));
-      HIPCHK(launch_finalize(g, d, n, nullptr, nullptr, st));
+      HIPCHK(launch_finalize(g, d, n, nullptr, nullptr, ResTry{}, st));
     }
     return TEUK_OK;
   };
@@ -1828,26 +1859,31 @@ int teuk_solve_noalloc_wait(const teuk_params *p, const double *r_c, const doubl
   if (nsteps < (1 << 28) && resident_shape(p->N, p->M, device_cus(), sh)) {
     HIPCHK(launch_init_res(g, d, st));
     int gate = 0;
-    for (int done = 0; done < nsteps; done += kRing, gate ^= 1) {
-      const int n = std::min(kRing, nsteps - done);
-      if (has_src) HIPCHK(launch_source(g, d, 0, n, true, st));
-      rc = resident_launch(
-          st,
-          [&]() {
-            return launch_resident(g, d, p->integrator, has_src, sh, ResSpan{0, p->N, 0, p->N, d.U, d.D, nullptr, 0}, n,
-                                   nsteps, d.ctl->gate + gate, res_wait_ticks(wait), st);
-          },
-          false);
-      if (rc) return rc;
-      HIPCHK(launch_finalize(g, d, n, d.ctl->gate + gate, d.ctl->gate + (gate ^ 1), st));
+    for (int missing = nsteps; missing > 0;) {   // (again for steps of launches that stepped aside)
+      for (int done = 0; done < missing; done += kRing, gate ^= 1) {
+        const int n = std::min(kRing, missing - done);
+        const ResTry t = res_try(wait, kResPatience, false);
+        if (has_src) HIPCHK(launch_source(g, d, 0, n, true, st));
+        rc = resident_launch(
+            st,
+            [&]() {
+              return launch_resident(g, d, p->integrator, has_src, sh, ResSpan{0, p->N, 0, p->N, d.U, d.D, nullptr, 0},
+                                     n, nsteps, d.ctl->gate + gate, t.limit, st);
+            },
+            false);
+        if (rc) return rc;
+        HIPCHK(launch_finalize(g, d, n, d.ctl->gate + gate, d.ctl->gate + (gate ^ 1), t, st));
+      }
+      HIPCHK(hipStreamSynchronize(st));
+      HIPCHK(hipMemcpy(&c, d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+      missing = nsteps - c.k;
+      if (c.tries.fail) break;
     }
-    HIPCHK(hipStreamSynchronize(st));
     if (ResidentChain *chain = resident_chain(st)) {
       std::lock_guard<std::mutex> hold_chain(chain->lock);
       chain->unrecorded = false;   // (waited for above)
     }
-    HIPCHK(hipMemcpy(&c, d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
-    if (c.fail && (rc = stage_chunks(nsteps - c.k))) return rc;
+    if (nsteps > 0 && c.tries.fail && (rc = stage_chunks(nsteps - c.k))) return rc;
   } else if ((rc = stage_chunks(nsteps))) {
     return rc;
   }

@@ -69,11 +69,28 @@ struct Grid {
 };
 
 // Gate of a resident launch (teuk_resident.inc): blocks that have arrived,
-// and 0 undecided, 1 the launch runs, 2 it gave up before changing anything.
+// and 0 undecided, 1 the launch runs, 2 it steps aside, changing nothing.
 // Two per owner, used in turn: the finalize of a launch clears the other one.
 struct ResGate {
   int arrived;
   int decision;
+};
+
+// How a solve's resident launches fared (written between them, k_finalize;
+// the host sets it back).
+struct ResTries {
+  int fail;            // they have waited too long in a row: later ones do nothing
+                       // until the host has run the missing steps
+  int aside;           // launches in a row that stepped aside
+  long long waited;    // ticks those waited
+  int cur;             // segments: the fields are in 0 the state U, 1 the state D
+  int asides;          // launches that stepped aside in all
+};
+// A launch's first wait before it steps aside, the waits in a row after which
+// it is not tried again (ticks), and whether its steps change U and D's places.
+struct ResTry {
+  long long limit, budget;
+  int flip;
 };
 
 // The most reads of a neighbour's flag in one wait, about a microsecond each.
@@ -86,8 +103,7 @@ struct Ctl {
   int status;          // 0 ok; bit 0: non-finite Psi at the extraction column,
                        // bit 1: the whole-field sentinel fired (see kGrowthLimit),
                        // bit 2: a resident launch stopped half way (its fields are no state)
-  int fail;            // a resident launch gave up: later ones do nothing until
-                       // the host has run the missing steps
+  ResTries tries;
   unsigned ended;      // blocks of the current record launch that have ended
   int reads;           // a resident launch's reads of a neighbour's flag in one wait (kResReads)
   double timer;        // solver time, advanced by repeated addition (body.cu:214)
@@ -180,7 +196,7 @@ struct ResBlock {
   int strip, C, B;     // block `strip` of the member's B blocks
 };
 // The columns [s0, s1) of a launch, those of them it stores ([v0, v1), into
-// `out`), its plane for the coefficient values, the launch before it in the
+// `out` from U, or from there into U where ResTries::cur says so), its plane for the coefficient values, the launch before it in the
 // same steps (or null) and its first block's flags.
 struct ResSpan {
   int s0, s1, v0, v1;
@@ -231,10 +247,23 @@ TEUK_HD constexpr size_t res_lds_bytes(int M, int C, int CP) {
 TEUK_HD constexpr int res_least_tile(int M, int CP) { return CP >= 4 ? ((res_groups(M, CP) * (CP / 2) + 11) & ~7) : 8; }
 constexpr size_t kResLdsMax = 163840 - 512;   // a CU's LDS less the kernel's static part
 constexpr int kResCP[5] = {1, 2, 4, 6, 8};
-// A launch's longest wait for all of its blocks to be on the GPU (s), unless
-// one is given, and the longest it takes: a launch must end in bounded time,
-// also where two processes each hold CUs that the other waits for.
+// Launches' longest wait in a row for all of their blocks to be on the GPU (s),
+// unless one is given, and the longest taken: it must end in bounded time.
 constexpr double kResWait = 0.25, kResWaitMost = 60.0;
+// The first wait of a launch.  Two processes' launches that each hold CUs which
+// the other waits for must not both wait on: one steps aside, the other runs,
+// and the first's steps are taken by the launches queued behind it.  The wait
+// is drawn from 0.5 to 1.5 times this, so that one is first, and doubles with
+// each launch in a row that stepped aside, up to 6.4 ms, so that the launches
+// of others (0.3 to 1.2 ms) are also waited out.  (A first wait of 0: the first
+// try steps aside whatever happens, the next ones wait as others do.)
+constexpr double kResPatience = 1e-4;
+TEUK_HD long long res_patience(long long limit, int aside) {
+  if (limit <= 0 && aside > 0) limit = 10000;
+  const long long most = limit > 640000 ? limit : 640000;
+  const long long w = limit << (aside < 20 ? aside : 20);
+  return w < most ? w : most;
+}
 // That wait in the GPU's 100 MHz ticks; 0: it does not wait.
 inline long long res_wait_ticks(double seconds) {
   if (!(seconds > 0.0)) return 0;
@@ -355,9 +384,9 @@ hipError_t launch_source_at(const Grid &g, const DevState &d, int kstep, hipStre
 hipError_t launch_stage(const Grid &g, const DevState &d, int integrator, int stage,
                         bool has_src, int k_rel, Tiling t, hipStream_t s);
 // gate: the gate of the resident launch that ran the steps (the other of its
-// pair, or all `others` of it, is cleared), or null.
-hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, hipStream_t s,
-                           int others = 1);
+// pair, or all `others` of it, is cleared) and what it waited, or null.
+hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, ResTry t,
+                           hipStream_t s, int others = 1);
 // The ABI's four real planes to the device's two planes of pairs and back
 // (in and out apart).
 hipError_t launch_fields_join(const double *in, double *out, size_t NM, hipStream_t s);
@@ -398,7 +427,7 @@ hipError_t launch_stage_rows(const Grid &g, const DevState &d, int integrator, i
 template <int R>
 hipError_t launch_stage_batch_rows(const BatchTile *tiles, int ntiles, int integrator, int stage, int k_rel,
                                    dim3 block, int wpe, hipStream_t s);
-hipError_t launch_finalize_batch(const SolveDesc *descs, int nsolves, int n, ResGate *gate, ResGate *other,
+hipError_t launch_finalize_batch(const SolveDesc *descs, int nsolves, int n, ResGate *gate, ResGate *other, ResTry t,
                                  hipStream_t s);
 // The sentinel of every member still running before the chunk's finalize.
 hipError_t launch_sentinel_batch(const SolveDesc *descs, int nsolves, hipStream_t s);

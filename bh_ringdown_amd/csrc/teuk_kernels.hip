@@ -96,14 +96,22 @@ constexpr int kFinTerms = 80;
 constexpr int kFinThreads = 512;
 
 __device__ __forceinline__ void finalize_solve(const Grid &g, const Ext &ext_in, Ctl *ctl_in, int n,
-                                               const ResGate *gate, ResGate *other, int others, int first) {
+                                               const ResGate *gate, ResGate *other, int others, const ResTry &tr,
+                                               int first) {
   __shared__ double terms[kFinTerms][15];
   const int M = g.M, t = threadIdx.x;
   if (gate) {
     if (first && t < others) other[t].arrived = other[t].decision = 0;
-    // the launch gave up, or an earlier one had: no step was taken
+    // the launch stepped aside, or did nothing as an earlier one's waits were
+    // too long: no step was taken
     if (gate->decision != 1) {
-      if (first && t == 0) ctl_in->fail = 1;
+      if (first && t == 0) {
+        ResTries &r = ctl_in->tries;
+        r.waited += res_patience(tr.limit, r.aside);
+        r.aside++;
+        r.asides++;
+        if (r.waited >= tr.budget) r.fail = 1;
+      }
       return;
     }
   }
@@ -171,6 +179,11 @@ __device__ __forceinline__ void finalize_solve(const Grid &g, const Ext &ext_in,
     double timer = timer0;
     for (int i = 0; i < n; i++) timer = __dadd_rn(timer, dt);
     ctl->ended = 0;
+    if (gate) {
+      ctl->tries.aside = 0;
+      ctl->tries.waited = 0;
+      if (tr.flip) ctl->tries.cur ^= 1;
+    }
     ctl->k = k0 + n;
     ctl->timer = timer;
     ctl->nrec = r_hi > ctl->nrec ? r_hi : ctl->nrec;
@@ -178,20 +191,20 @@ __device__ __forceinline__ void finalize_solve(const Grid &g, const Ext &ext_in,
 }
 
 __global__ __launch_bounds__(kFinThreads) void k_finalize(Grid g, Ext ext, Ctl *ctl, int n, const ResGate *gate,
-                                                          ResGate *other, int others) {
-  finalize_solve(g, ext, ctl, n, gate, other, others, blockIdx.x == 0);
+                                                          ResGate *other, int others, ResTry tr) {
+  finalize_solve(g, ext, ctl, n, gate, other, others, tr, blockIdx.x == 0);
 }
 
 // blockIdx.y = member; a member closes at its scheduled step count.
 __global__ __launch_bounds__(kFinThreads) void k_finalize_batch(const SolveDesc *__restrict__ descs, int n,
-                                                                const ResGate *gate, ResGate *other) {
+                                                                const ResGate *gate, ResGate *other, ResTry tr) {
   const SolveDesc &sd = descs[blockIdx.y];
   const bool first = blockIdx.x == 0 && blockIdx.y == 0;
   const int left = sd.nt - sd.d.ctl->k;
   const int n_eff = n < left ? n : left;
   if (gate && first && threadIdx.x == 0) other->arrived = other->decision = 0;
   if (n_eff <= 0) return;
-  finalize_solve(sd.g, sd.d.ext, sd.d.ctl, n_eff, gate, other, 0, blockIdx.x == 0);
+  finalize_solve(sd.g, sd.d.ext, sd.d.ctl, n_eff, gate, other, 0, tr, blockIdx.x == 0);
 }
 
 // Whole-field sentinel (no counterpart in the reference, which checks
@@ -352,11 +365,11 @@ static unsigned finalize_blocks(int n, int Fr) {
   return (unsigned)std::min(most, 2 * kRing);
 }
 
-hipError_t launch_finalize_batch(const SolveDesc *descs, int nsolves, int n, ResGate *gate, ResGate *other,
+hipError_t launch_finalize_batch(const SolveDesc *descs, int nsolves, int n, ResGate *gate, ResGate *other, ResTry t,
                                  hipStream_t s) {
   if (nsolves <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_finalize_batch, dim3(finalize_blocks(n, 1), nsolves), dim3(kFinThreads), 0, s, descs, n, gate,
-                     other);
+                     other, t);
   return hipGetLastError();
 }
 
@@ -369,10 +382,10 @@ hipError_t launch_source_batch(const SolveDesc *descs, int nsolves, int max_cell
   return hipGetLastError();
 }
 
-hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, hipStream_t s,
-                           int others) {
+hipError_t launch_finalize(const Grid &g, const DevState &d, int n, ResGate *gate, ResGate *other, ResTry t,
+                           hipStream_t s, int others) {
   hipLaunchKernelGGL(k_finalize, dim3(finalize_blocks(n, g.Fr)), dim3(kFinThreads), 0, s, g, d.ext, d.ctl, n, gate,
-                     other, others);
+                     other, others, t);
   return hipGetLastError();
 }
 

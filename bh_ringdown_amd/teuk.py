@@ -77,7 +77,8 @@ EXPORTS = [
     "teuk_batch_remove", "teuk_batch_set_tiling", "teuk_batch_step", "teuk_batch_sync", "teuk_batch_info",
     "teuk_source_coeffs", "teuk_source_patch", "teuk_grid_half", "teuk_create_staggered",
     "teuk_trajectory_schedule_staggered", "teuk_status", "teuk_solve_noalloc", "teuk_batch_set_cache_groups",
-    "teuk_ot_transition", "teuk_set_resident_wait", "teuk_set_exchange_reads", "teuk_resident", "teuk_set_theta_rows", "teuk_batch_set_theta_rows",
+    "teuk_ot_transition", "teuk_set_resident_wait", "teuk_set_exchange_reads",
+    "teuk_set_resident_patience", "teuk_resident", "teuk_set_theta_rows", "teuk_batch_set_theta_rows",
     "teuk_batch_set_resident", "teuk_solve_noalloc_wait",
 ]
 
@@ -137,6 +138,7 @@ def lib():
         "teuk_set_theta_rows": ([vp, ctypes.c_int], ctypes.c_int),
         "teuk_resident": ([vp, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
         "teuk_set_resident_wait": ([vp, ctypes.c_double], ctypes.c_int),
+        "teuk_set_resident_patience": ([vp, ctypes.c_double], ctypes.c_int),
         "teuk_set_exchange_reads": ([vp, ctypes.c_int], ctypes.c_int),
         "teuk_batch_set_theta_rows": ([vp, ctypes.c_int], ctypes.c_int),
         "teuk_batch_set_resident": ([vp, ctypes.c_int], ctypes.c_int),
@@ -358,8 +360,12 @@ class Solver:
             _check(lib().teuk_set_theta_rows(self._h, int(theta_rows)), "teuk_set_theta_rows")
 
     def set_resident_wait(self, seconds):
-        """Longest wait of a resident launch for its blocks (teuk_set_resident_wait)."""
+        """Longest wait in a row of resident launches for their blocks (teuk_set_resident_wait)."""
         _check(lib().teuk_set_resident_wait(self._h, float(seconds)), "teuk_set_resident_wait")
+
+    def set_resident_patience(self, seconds):
+        """First wait of a resident launch before it steps aside (teuk_set_resident_patience)."""
+        _check(lib().teuk_set_resident_patience(self._h, float(seconds)), "teuk_set_resident_patience")
 
     def set_exchange_reads(self, reads):
         """Reads of a neighbour's flag in one wait of a resident launch (teuk_set_exchange_reads)."""

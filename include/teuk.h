@@ -174,7 +174,8 @@ int teuk_read_psi(teuk_solver *s, int first, int max, double *psi, int *n);
  * stage-kernel launches (or each resident launch, of up to 32 steps) with a
  * pair of HIP events on the solver stream.  teuk_timing returns the number of
  * timed stages and their summed duration in milliseconds (without those of a
- * resident launch that gave up, and of the ones waited for together with it). */
+ * resident launch that stepped aside, and of the ones waited for together with
+ * it). */
 int teuk_enable_timing(teuk_solver *s, int on);
 int teuk_timing(teuk_solver *s, long long *launches, double *ms);
 
@@ -205,12 +206,18 @@ int teuk_set_theta_rows(teuk_solver *s, int rows);
  * kernels (teuk_set_tiling, teuk_set_theta_rows): grids of up to about a
  * million points whole, larger ones in segments of rho columns, one after
  * the other, where that is faster.  Such a launch needs all of its blocks on
- * the GPU at once.  If it does not get them within `seconds` (0.25 by default; 0: it
- * never waits; at most 60, which larger values are taken as), because another
- * process holds the CUs, it changes nothing, and its steps and all later ones
- * are run by the stage kernels.  A launch that members of a batch share
- * waits as long as the shortest of their waits.  Results do not depend on it. */
+ * the GPU at once.  One that does not get them soon, because another process
+ * holds CUs, steps aside without having changed anything, and its steps are
+ * taken by later ones.  If launches in a row wait for `seconds` in all (0.25 by
+ * default; 0: they never wait; at most 60, which larger values are taken as),
+ * the steps and all later ones are run by the stage kernels.  A launch that
+ * members of a batch share waits as long as the shortest of their waits.
+ * Results do not depend on it. */
 int teuk_set_resident_wait(teuk_solver *s, double seconds);
+/* The first of those waits: 100 us by default, at most 60 s.  Each launch draws
+ * its own from 0.5 to 1.5 times this, and the next waits are twice as long, up
+ * to 6.4 ms.  0: every launch's first try steps aside, for tests. */
+int teuk_set_resident_patience(teuk_solver *s, double seconds);
 /* Blocks of a resident launch wait for each other's edge columns.  A wait ends
  * after about `reads` reads of the neighbour's flag (2^22 by default, some
  * seconds of them), which it reaches only if a block has stopped; the solve

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from bh_ringdown_amd import teuk
-from tests.test_gpu_resident import setup, start
+from tests.test_gpu_resident import oracle, setup, start
 
 pytestmark = pytest.mark.gpu
 
@@ -92,6 +92,60 @@ def test_resident_of_members():
             assert np.array_equal(s.get_fields(), one.get_fields())
     b.close()
     assert [s.resident() for s in solvers] == [True, True, False]      # alone again
+    for s in solvers:
+        s.close()
+
+
+@pytest.mark.parametrize("N,M,integrator,patience", [
+    (1024, 32, 1, 0.0), (6080, 40, 0, 0.0), (16384, 64, 1, 0.0), (6144, 128, 0, 0.0), (32768, 64, 1, 0.0),
+    (32768, 64, 0, 1e-8), (16384, 128, 1, 1e-8), (32768, 64, 1, 1e-8),
+])
+def test_launches_that_step_aside_are_tried_again(N, M, integrator, patience):
+    """With no first wait every launch's first try steps aside; with a first
+    wait of 0.5 to 1.5 ticks every other segment's, also after segments that
+    have run.  The steps are taken by later launches."""
+    print(f"step aside {N}x{M} integrator {integrator} patience {patience}", flush=True)
+    parts = (1, 1, 1, 1, 1, 1, 2, 33, 6)
+    steps = sum(parts)
+    p, u0, rows = setup(N, M, integrator, 2, steps, N // 3, True)
+    uo, psio, ho, _ = oracle(p, u0, rows, steps)
+    with start(p, u0, rows, steps) as s:
+        s.set_resident_patience(patience)
+        s.enable_timing(True)
+        for n in parts:
+            s.step(n)
+            assert s.progress()[0] == s.p.nsteps() - s.remaining()
+        assert s.timing()[0] < (3, 4)[integrator] * steps      # those tried again are not timed
+        assert s.resident() and s.progress()[0] == steps
+        assert np.array_equal(s.get_fields(), uo) and np.array_equal(s.psi(), psio)
+        assert np.array_equal(s.output()["h"], ho)
+    with start(p, u0, rows, steps) as s:                        # queued at once
+        s.set_resident_patience(patience)
+        s.step(3)
+        s.step(steps - 3)
+        s.sync()
+        assert s.resident() and s.progress()[0] == steps
+        assert np.array_equal(s.get_fields(), uo) and np.array_equal(s.output()["h"], ho)
+
+
+def test_batch_launches_that_step_aside_are_tried_again():
+    specs = [setup(N, M, 1, 2, 70, seed=i) for i, (N, M) in enumerate([(1024, 32), (4096, 32), (512, 72), (8192, 64)])]
+    ref = []
+    for p, u0, _ in specs:
+        with start(p, u0, None, 70) as s:
+            s.step(70)
+            s.sync()
+            ref.append((s.get_fields(), s.output()["h"]))
+    b, solvers = batch_of(specs, 70)
+    solvers[2].set_resident_patience(0.0)
+    for n in (5, 40, 25):
+        b.step(n)
+        b.sync()
+    assert b.info()["active"] == 0
+    for s, (u, h) in zip(solvers, ref):
+        assert s.resident() and s.progress()[0] == 70
+        assert np.array_equal(s.get_fields(), u) and np.array_equal(s.output()["h"], h)
+    b.close()
     for s in solvers:
         s.close()
 

@@ -37,6 +37,6 @@ def test_scratch_of_resident_kernels(cp, tmp_path):
     found = kernels(cp, str(tmp_path))
     assert len(found) >= 12
     for key, scratch in found.items():
-        # (up to 16 spilled registers: rows that are not built in, and RK4's 32-row sweeps of four columns)
-        most = 64 if key[2] == 0 or (cp == 8 and key[2] == 32) else 0
+        # (up to 20 spilled registers: rows that are not built in, and RK4's 32-row sweeps of four columns)
+        most = 80 if key[2] == 0 or (cp == 8 and key[2] == 32) else 0
         assert scratch <= most, (key, scratch)
